@@ -19,7 +19,7 @@ import torch
 class DGRollout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u0: torch.Tensor, solver, dt: float, nsteps: int, snapshots: int):
-        solver.set_state(u0.detach().cpu().numpy().astype(np.float64))
+        solver.set_state(u0.detach().cpu().numpy().astype(np.float64, copy=False))
         solver.adjoint_forward(dt, nsteps, snapshots)
         un = solver.get_state()
         ctx.solver = solver
@@ -30,7 +30,7 @@ class DGRollout(torch.autograd.Function):
         if grad_out.is_cuda:  # device-resident reverse sweep: no host round trip of the adjoints
             lam = grad_out.detach().to(torch.float64).contiguous()
             return ctx.solver.adjoint_backward_device(lam).to(grad_out.dtype), None, None, None, None
-        lam0 = ctx.solver.adjoint_backward(grad_out.detach().cpu().numpy().astype(np.float64))
+        lam0 = ctx.solver.adjoint_backward(grad_out.detach().cpu().numpy().astype(np.float64, copy=False))
         return torch.from_numpy(lam0).to(dtype=grad_out.dtype, device=grad_out.device), None, None, None, None
 
 

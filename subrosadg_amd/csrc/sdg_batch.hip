@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <climits>
 #include <cstdint>
@@ -23,6 +24,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/sdg.h"
@@ -460,6 +462,42 @@ __global__ __launch_bounds__(kThreads) void batchDtKernel(const double* U, const
   out[vd.e_base + e] = best;
 }
 
+// One problem's elements of one variant between the reference layout (element blocks [mode][variable]
+// at coff, phi coefficients) and the device panels ([variable][mode], psi coefficients; panel and coff
+// start at the problem's first element): c_phi = L^-T c_psi, c_psi = L^T c_phi. One thread per (element,
+// mode) moves the four variables, so that the stores of the reference layout are 32 contiguous bytes.
+__global__ __launch_bounds__(kThreads) void batchToReferenceKernel(const double* panel, const int64_t* coff, int64_t n,
+                                                                   int nb, const double* Li, double* out) {
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (idx >= n * nb) return;
+  const int64_t e = idx / nb;
+  const int i = static_cast<int>(idx % nb);
+  double acc[NV] = {0.0, 0.0, 0.0, 0.0};
+  for (int j = i; j < nb; j++) {
+    const double l = Li[j * nb + i];
+    for (int v = 0; v < NV; v++) acc[v] += l * panel[(e * NV + v) * nb + j];
+  }
+  double* o = out + coff[e] + static_cast<int64_t>(i) * NV;
+  for (int v = 0; v < NV; v++) o[v] = acc[v];
+}
+__global__ __launch_bounds__(kThreads) void batchFromReferenceKernel(const double* in, const int64_t* coff, int64_t n,
+                                                                     int nb, const double* Lc, double* U, double* Un) {
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (idx >= n * nb) return;
+  const int64_t e = idx / nb;
+  const int j = static_cast<int>(idx % nb);
+  const double* c = in + coff[e];
+  double acc[NV] = {0.0, 0.0, 0.0, 0.0};
+  for (int i = j; i < nb; i++) {
+    const double l = Lc[i * nb + j];
+    for (int v = 0; v < NV; v++) acc[v] += l * c[i * NV + v];
+  }
+  for (int v = 0; v < NV; v++) {
+    U[(e * NV + v) * nb + j] = acc[v];
+    Un[(e * NV + v) * nb + j] = acc[v];
+  }
+}
+
 }  // namespace batch
 }  // namespace sdg
 
@@ -489,7 +527,13 @@ struct sdg_batch {
   int8_t* fflag = nullptr;
   // per variant the reference element's Cholesky factor L of Mref (row-major) and L^-1: the
   // device state is in psi = L^-1 phi coefficients, c_psi = L^T c_phi
-  std::vector<double> chol[sdg::batch::kVariants], chol_inv[sdg::batch::kVariants];
+  double *chol[sdg::batch::kVariants] = {}, *chol_inv[sdg::batch::kVariants] = {};
+  // state transfers: per device element its offset in its problem's reference layout, per problem
+  // the first element and the count in each variant, and a buffer for the largest problem
+  int64_t* coff = nullptr;
+  std::vector<std::array<std::pair<int64_t, int64_t>, sdg::batch::kVariants>> range;
+  std::vector<int64_t> ncoeff;  // coefficients of each problem
+  double* io = nullptr;
   void* T[2] = {nullptr, nullptr};
   sdg::batch::VariantDev* dvar = nullptr;
   sdg::batch::WorkItem* ditems = nullptr;
@@ -759,8 +803,11 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
   // variants present and their element ranges (problem-major within a variant)
   b->emap.resize(count);
   b->coeff_off.resize(count);
+  b->range.resize(count);
+  b->ncoeff.resize(count);
   for (int p = 0; p < count; p++) {
     const sdg::MixedMesh& m = *b->meshes[p];
+    for (int v = 0; v < sdg::batch::kVariants; v++) b->range[p][v] = {b->var[v].E, 0};
     b->emap[p].resize(m.elements);
     b->coeff_off[p].resize(m.elements);
     int64_t off = 0;
@@ -783,6 +830,8 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
       b->coeff_off[p][e] = off;
       off += static_cast<int64_t>(r.nb) * 4;
     }
+    for (int v = 0; v < sdg::batch::kVariants; v++) b->range[p][v].second = b->var[v].E - b->range[p][v].first;
+    b->ncoeff[p] = off;
   }
   // re-index variant elements problem-major: index = (running count at creation) already is
   int64_t eb = 0, ub = 0, tb = 0, fb = 0;
@@ -819,8 +868,7 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
       if (std::fabs(x - 1.0) < 1e-12) x = 1.0;
       one_phi[k] = x;
     }
-    b->chol[v] = r.mass_chol;
-    b->chol_inv[v] = r.mass_chol_inverse;
+    if (bupload(b, r.mass_chol, &b->chol[v]) || bupload(b, r.mass_chol_inverse, &b->chol_inv[v])) return bail(SDG_E_NOMEM);
     V.one.assign(r.nb, 0.0);  // c_psi = L^T c_phi
     for (int j2 = 0; j2 < r.nb; j2++) {
       double x = 0.0;
@@ -842,6 +890,7 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
   }
   std::vector<double> ginv(static_cast<size_t>(eb) * 4), detj(eb), me(eb);
   std::vector<double> fnrm(static_cast<size_t>(face_off[count]) * 2), fjw(static_cast<size_t>(face_off[count]) * sdg::batch::kMaxNfq, 0.0);
+  std::vector<int64_t> coff(eb);
   std::vector<int> pid(eb), fid(fb);
   std::vector<int64_t> fnb(fb);
   std::vector<int8_t> fflag(fb);
@@ -878,6 +927,7 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
       detj[ge] = m.detj[e];
       me[ge] = m.min_edge[e];
       pid[ge] = p;
+      coff[ge] = b->coeff_off[p][e];
       for (int s = 0; s < V.nf; s++) {
         const int f = m.elem_face[static_cast<size_t>(e) * 4 + s];
         const int side = m.elem_side[static_cast<size_t>(e) * 4 + s];
@@ -942,7 +992,8 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
   const size_t tbytes = b->mixed ? sizeof(float) : sizeof(double);
   void *t0 = nullptr, *t1 = nullptr;
   if (bupload(b, dv, &b->dvar) || bupload(b, ginv, &b->ginv) || bupload(b, detj, &b->detj) || bupload(b, me, &b->min_edge) ||
-      bupload(b, pid, &b->pid) || bupload(b, fnb, &b->fnb) || bupload(b, fid, &b->fid) || bupload(b, fflag, &b->fflag) ||
+      bupload(b, pid, &b->pid) || bupload(b, coff, &b->coff) ||
+      balloc(b, static_cast<size_t>(*std::max_element(b->ncoeff.begin(), b->ncoeff.end())), &b->io) || bupload(b, fnb, &b->fnb) || bupload(b, fid, &b->fid) || bupload(b, fflag, &b->fflag) ||
       bupload(b, fnrm, &b->fnrm) || bupload(b, fjw, &b->fjw) || balloc(b, static_cast<size_t>(ub), &b->U) ||
       balloc(b, static_cast<size_t>(ub), &b->Un) || balloc(b, static_cast<size_t>(count), &b->dt) ||
       balloc(b, static_cast<size_t>(count) * 6, &b->mix) || balloc(b, static_cast<size_t>(eb), &b->dtbuf) ||
@@ -988,43 +1039,19 @@ void sdg_batch_destroy(sdg_batch* b) {
 
 int sdg_batch_set_state(sdg_batch* b, int p, const double* coeff) {
   if (!b || !coeff || p < 0 || p >= b->nprob) return bfail(b, SDG_E_INVALID, "sdg_batch_set_state: bad argument");
-  const sdg::MixedMesh& m = *b->meshes[p];
   updateMix(b, p, coeff);
-  // scatter into the device layout of each variant: the problem's elements of one variant are
-  // contiguous there, so one copy per variant
-  int64_t lo[sdg::batch::kVariants], hi[sdg::batch::kVariants];
+  BHIP(b, hipMemcpyAsync(b->io, coeff, static_cast<size_t>(b->ncoeff[p]) * sizeof(double), hipMemcpyHostToDevice, b->stream));
   for (int v = 0; v < sdg::batch::kVariants; v++) {
-    lo[v] = INT64_MAX;
-    hi[v] = -1;
-  }
-  for (int64_t e = 0; e < m.elements; e++) {
-    const auto [v, k] = b->emap[p][e];
-    lo[v] = std::min(lo[v], k);
-    hi[v] = std::max(hi[v], k);
-  }
-  std::vector<std::vector<double>> host(sdg::batch::kVariants);
-  for (int v = 0; v < sdg::batch::kVariants; v++)
-    if (hi[v] >= 0) host[v].assign(static_cast<size_t>(hi[v] - lo[v] + 1) * 4 * b->var[v].nb, 0.0);
-  for (int64_t e = 0; e < m.elements; e++) {
-    const auto [v, k] = b->emap[p][e];
+    const auto [lo, n] = b->range[p][v];
+    if (n == 0) continue;
     const auto& V = b->var[v];
-    double* panel = &host[v][static_cast<size_t>(k - lo[v]) * 4 * V.nb];
-    const double* c = coeff + b->coeff_off[p][e];
-    const std::vector<double>& Lc = b->chol[v];  // c_psi[j] = sum_{i >= j} L[i][j] c_phi[i]
-    for (int vv = 0; vv < 4; vv++)
-      for (int j = 0; j < V.nb; j++) {
-        double acc = 0.0;
-        for (int i = j; i < V.nb; i++) acc += Lc[static_cast<size_t>(i) * V.nb + j] * c[i * 4 + vv];
-        panel[static_cast<size_t>(vv) * V.nb + j] = acc;
-      }
+    const int64_t off = V.u_base + lo * 4 * V.nb;
+    hipLaunchKernelGGL(sdg::batch::batchFromReferenceKernel,
+                       dim3(static_cast<unsigned>((n * V.nb + sdg::batch::kThreads - 1) / sdg::batch::kThreads)),
+                       dim3(sdg::batch::kThreads), 0, b->stream, b->io, b->coff + V.e_base + lo, n, V.nb, b->chol[v],
+                       b->U + off, b->Un + off);
   }
-  for (int v = 0; v < sdg::batch::kVariants; v++) {
-    if (hi[v] < 0) continue;
-    const size_t off = static_cast<size_t>(b->var[v].u_base + lo[v] * 4 * b->var[v].nb);
-    BHIP(b, hipMemcpyAsync(b->U + off, host[v].data(), host[v].size() * sizeof(double), hipMemcpyHostToDevice, b->stream));
-    BHIP(b, hipMemcpyAsync(b->Un + off, host[v].data(), host[v].size() * sizeof(double), hipMemcpyHostToDevice, b->stream));
-  }
-  BHIP(b, hipStreamSynchronize(b->stream));
+  BHIP(b, hipGetLastError());
   BHIP(b, hipMemcpyAsync(b->mix + static_cast<size_t>(p) * 6, &b->mixh[static_cast<size_t>(p) * 6], 6 * sizeof(double),
                          hipMemcpyHostToDevice, b->stream));
   b->has_state[p] = 1;
@@ -1039,25 +1066,22 @@ int sdg_batch_set_state(sdg_batch* b, int p, const double* coeff) {
   return SDG_OK;
 }
 
+// The conversion runs on the device and only problem p crosses to the host: copying every problem's
+// state and converting on the host took 17 ms a call with 48 problems of up to 96^2 cells.
 int sdg_batch_get_state(sdg_batch* b, int p, double* coeff) {
   if (!b || !coeff || p < 0 || p >= b->nprob) return bfail(b, SDG_E_INVALID, "sdg_batch_get_state: bad argument");
-  const sdg::MixedMesh& m = *b->meshes[p];
-  std::vector<double> host(static_cast<size_t>(b->totalU));
-  BHIP(b, hipMemcpyAsync(host.data(), b->U, host.size() * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-  BHIP(b, hipStreamSynchronize(b->stream));
-  for (int64_t e = 0; e < m.elements; e++) {
-    const auto [v, k] = b->emap[p][e];
+  for (int v = 0; v < sdg::batch::kVariants; v++) {
+    const auto [lo, n] = b->range[p][v];
+    if (n == 0) continue;
     const auto& V = b->var[v];
-    const double* panel = &host[static_cast<size_t>(V.u_base + k * 4 * V.nb)];
-    double* c = coeff + b->coeff_off[p][e];
-    const std::vector<double>& Li = b->chol_inv[v];  // c_phi[i] = sum_{j >= i} (L^-1)[j][i] c_psi[j]
-    for (int vv = 0; vv < 4; vv++)
-      for (int i = 0; i < V.nb; i++) {
-        double acc = 0.0;
-        for (int j = i; j < V.nb; j++) acc += Li[static_cast<size_t>(j) * V.nb + i] * panel[static_cast<size_t>(vv) * V.nb + j];
-        c[i * 4 + vv] = acc;
-      }
+    hipLaunchKernelGGL(sdg::batch::batchToReferenceKernel,
+                       dim3(static_cast<unsigned>((n * V.nb + sdg::batch::kThreads - 1) / sdg::batch::kThreads)),
+                       dim3(sdg::batch::kThreads), 0, b->stream, b->U + V.u_base + lo * 4 * V.nb, b->coff + V.e_base + lo,
+                       n, V.nb, b->chol_inv[v], b->io);
   }
+  BHIP(b, hipGetLastError());
+  BHIP(b, hipMemcpyAsync(coeff, b->io, static_cast<size_t>(b->ncoeff[p]) * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+  BHIP(b, hipStreamSynchronize(b->stream));
   return SDG_OK;
 }
 
