@@ -195,11 +195,12 @@ __device__ __forceinline__ double faceStateVjpDir(const Phys& ph, const double* 
 
 // ---- kernel 1: volume part ----------------------------------------------------------------------
 template <int D, int NB, int NQ, int NF, int NFQ, int VISC>
-__global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
+__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjVolumeMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
   constexpr int NV = LD::NV, NG = LD::NG, EPB = LD::EPB, NAQ = LD::NAQ;
   constexpr int NBk = LD::NBk, NBm = LD::NBm, NQm = LD::NQm, NQk = r4(NQ), NAQm = LD::NAQm;
   constexpr int NBr = LD::NBr, NDQm = r16(NQ * D);
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
   constexpr int AJV = LD::AJ > 2 * NQm * 16 ? LD::AJ : 2 * NQm * 16;  // grad u_q and grad-bar_q
   static_assert(2 * NBr >= NQm, "u-bar_q reuses the lifting work area");
   __shared__ double sUq[NQm * 16];
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   double* sGq = sAJ;
   double* sLam = sRR;
   double* sMu = sRR + NBr * 16;
-  for (int idx = tid; idx < NBr * 16; idx += kThreads) {
+  for (int idx = tid; idx < NBr * 16; idx += NT) {
     const int b = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
     sLam[idx] = (b < NB && cc < EPB * NV && e < g.E) ? j.lam[(static_cast<int64_t>(e) * NV + v) * NB + b] : 0.0;
   }
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   const bool col_ok = c < EPB * NV && e_c < g.E;
   // mu = Mref^-1 lam / |J| (adjoint of M^-1 R) or lam
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     if (j.apply_minv) {
       tileAcc<double, NBm>(acc, op.minv, m0, sLam, 0, NBk, lane);
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   __syncthreads();
   // H-bar = Vf mu at the face slots -> HBM
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NAQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NAQm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NAQm>(acc, op.trace, m0, sMu, 0, NBk, lane);
 #pragma unroll
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   }
   // F-bar = Phi_grad mu at the (point, direction) rows
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NDQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NDQm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NDQm>(acc, j.op.gradT, m0, sMu, 0, NBk, lane);
     tileStore<double>(acc, sFb, m0, lane);
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   // grad-bar_q into sGb (behind grad u_q in sAJ)
   double* sUb = sRR;
   double* sGb = sAJ + NQm * 16;
-  for (int idx = tid; idx < 2 * EPB * NQ; idx += kThreads) {
+  for (int idx = tid; idx < 2 * EPB * NQ; idx += NT) {
     const int part = idx / (EPB * NQ), rem = idx % (EPB * NQ), le = rem / NQ, q = rem % NQ, e = e0 + le;
     if (e >= g.E) continue;
     double u[NV], gq[NG], G[D * D], fb[D * NV], Fb[D * NV];
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   const bool gok = c < EPB * NG && ge < g.E;
   const double idj = gok ? 1.0 / g.detj[ge] : 0.0;
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NBm>(acc, j.op.pinterpT, m0, sGb, 0, NQk, lane);
 #pragma unroll
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjVolumeMfma(Geo g, Phys ph, Stag
   }
   // U-bar (partial) = V^T u-bar_q -> HBM
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NBm>(acc, j.op.interpT, m0, sUb, 0, NQk, lane);
 #pragma unroll
@@ -408,11 +409,12 @@ __global__ __launch_bounds__(kThreads) void nsAdjFaceRevKernel(Geo g, Phys ph, S
 
 // ---- kernel 3: lifting terms --------------------------------------------------------------------
 template <int D, int NB, int NQ, int NF, int NFQ, int VISC>
-__global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
+__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjLiftMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
   constexpr int NV = LD::NV, NG = LD::NG, EPB = LD::EPB, NAQ = LD::NAQ;
   constexpr int NBk = LD::NBk, NBm = LD::NBm, NQm = LD::NQm, NQk = r4(NQ), NAQk = LD::NAQk, NAQm = LD::NAQm;
   constexpr int NBr = LD::NBr, NDQm = r16(NQ * D);
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
   __shared__ double sRt[NBr * 16];
   __shared__ double sRw[NBr * 16];
   __shared__ double sGb[NAQm * 16];
@@ -424,12 +426,12 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
   const int e0 = blockIdx.x * EPB;
-  zeroLds(sUQ, NQm * 16, tid);
-  for (int idx = tid; idx < NBr * 16; idx += kThreads) {
+  zeroLds<NT>(sUQ, NQm * 16, tid);
+  for (int idx = tid; idx < NBr * 16; idx += NT) {
     const int b = idx / 16, cc = idx % 16, le = cc / NG, r = cc % NG, e = e0 + le;
     sRt[idx] = (b < NB && cc < EPB * NG && e < g.E) ? j.RtV[(static_cast<int64_t>(e) * NG + r) * NB + b] : 0.0;
   }
-  for (int idx = tid; idx < NAQm * 16; idx += kThreads) {
+  for (int idx = tid; idx < NAQm * 16; idx += NT) {
     const int sl = idx / 16, cc = idx % 16, le = cc / NG, r = cc % NG, e = e0 + le;
     sGb[idx] = (sl < NAQ && cc < EPB * NG && e < g.E) ? j.GFb[(static_cast<int64_t>(e) * NG + r) * NAQ + sl] : 0.0;
   }
@@ -439,7 +441,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
   const double idj = gok ? 1.0 / g.detj[ge] : 0.0;
   // face-gradient adjoint -> R-bar_w (BR2) or R-bar_t (BR1); each lane updates its own entries
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NBm>(acc, j.op.ptraceT, m0, sGb, 0, NAQk, lane);
 #pragma unroll
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
   __syncthreads();
   // J-bar = Vf R-bar_t (+ Lf^T G-bar / |J|), A-bar = Vf R-bar_w
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NAQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NAQm; m0 += STEP) {
     acc_t<double> aj = zeroAcc<double>(), aa = zeroAcc<double>();
     tileAcc<double, NAQm>(aj, op.trace, m0, sRt, 0, NBk, lane);
     if (VISC == 2) {
@@ -476,7 +478,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
   }
   // Q-bar = -Phi_grad R-bar_w
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NDQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NDQm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NDQm>(acc, j.op.gradT, m0, sRw, 0, NBk, lane);
 #pragma unroll
@@ -485,7 +487,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
   }
   __syncthreads();
   // Q = u_q (x) (J^T)^-1 |J| w: u-bar_q[k] = sum_{a,b} Q-bar[(q,b)][(k,a)] G[a][b]
-  for (int idx = tid; idx < EPB * NQ * NV; idx += kThreads) {
+  for (int idx = tid; idx < EPB * NQ * NV; idx += NT) {
     const int le = idx / (NQ * NV), rem = idx % (NQ * NV), q = rem / NV, kv = rem % NV, e = e0 + le;
     if (e >= g.E) continue;
     const double jw = g.detj[e] * g.wq[q];
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
     sUQ[q * 16 + le * NV + kv] = s;
   }
   // A and J face terms -> adjoints of the own trace (Pown) and of the neighbour's trace (Qnb)
-  for (int idx = tid; idx < EPB * NAQ * NV; idx += kThreads) {
+  for (int idx = tid; idx < EPB * NAQ * NV; idx += NT) {
     const int le = idx / (NAQ * NV), rem = idx % (NAQ * NV), sl = rem / NV, kv = rem % NV, e = e0 + le;
     if (e >= g.E) continue;
     const int64_t es = static_cast<int64_t>(e) * NAQ + sl;
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
   const int le_c = c / NV, v_c = c % NV, e_c = e0 + le_c;
   const bool col_ok = c < EPB * NV && e_c < g.E;
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NBm>(acc, j.op.interpT, m0, sUQ, 0, NQk, lane);
 #pragma unroll
@@ -535,15 +537,16 @@ __global__ __launch_bounds__(kThreads) void nsAdjLiftMfma(Geo g, Phys ph, StageA
 
 // ---- kernel 4: gather the trace adjoints and apply Vf^T ---------------------------------------
 template <int D, int NB, int NQ, int NF, int NFQ>
-__global__ __launch_bounds__(kThreads) void nsAdjGatherMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
+__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjGatherMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
   constexpr int NV = D + 2, NAQ = NF * NFQ, EPB = 16 / NV;
   constexpr int NBm = r16(NB), NAQk = r4(NAQ);
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
   __shared__ double sUf[NAQk * 16];
   const MOps& op = g.op;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
   const int e0 = blockIdx.x * EPB;
-  for (int idx = tid; idx < NAQk * 16; idx += kThreads) {
+  for (int idx = tid; idx < NAQk * 16; idx += NT) {
     const int sl = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
     double x = 0.0;
     if (sl < NAQ && cc < EPB * NV && e < g.E) {
@@ -558,7 +561,7 @@ __global__ __launch_bounds__(kThreads) void nsAdjGatherMfma(Geo g, Phys ph, Stag
   const int le_c = c / NV, v_c = c % NV, e_c = e0 + le_c;
   const bool col_ok = c < EPB * NV && e_c < g.E;
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     tileAcc<double, NBm>(acc, op.face, m0, sUf, 0, NAQk, lane);
 #pragma unroll

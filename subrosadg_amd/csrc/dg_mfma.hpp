@@ -70,9 +70,19 @@ __device__ __forceinline__ void tileStore(const acc_t<TC>& acc, TC* Y, int m0, i
   for (int i = 0; i < 4; i++) Y[(m0 + Mfma<TC>::row(r, i)) * 16 + c] = acc[i];
 }
 
-template <typename TC>
+// Workgroup of a matrix-core kernel: one wavefront per 16-row tile of its tallest operator, at most
+// four. A tile is one wavefront's chain of matrix instructions, so further wavefronts only wait at
+// the barriers, and at one tile (quadrangles P3) the barriers cost nothing at all.
+template <int NB, int NQ, int NAQ>
+struct MfmaShape {
+  static constexpr int TILES = r16(NB > NQ ? (NB > NAQ ? NB : NAQ) : (NQ > NAQ ? NQ : NAQ)) / 16;
+  static constexpr int WAVES = TILES < 4 ? TILES : 4;
+  static constexpr int NT = 64 * WAVES, STEP = 16 * WAVES;
+};
+
+template <int NT, typename TC>
 __device__ __forceinline__ void zeroLds(TC* p, int n, int tid) {
-  for (int i = tid; i < n; i += kThreads) p[i] = TC(0);
+  for (int i = tid; i < n; i += NT) p[i] = TC(0);
 }
 
 // FP32 deviation of a coefficient from the reference state's (one expression for every producer
@@ -132,11 +142,11 @@ __device__ __forceinline__ double restoreEnergy(const StageArgs& a, double x, in
 // the current state; mixed mode: scratch, the update reads the FP64 state from HBM).
 // + the modal source residual of the last momentum component (Rsrc), before the update or the
 // residual output; the FP64 kernels only (the mixed mode refuses a source term)
-template <typename TC, int D, int NB, int EPB>
+template <typename TC, int D, int NB, int EPB, int NT>
 __device__ __forceinline__ void addSource(const Geo& g, const StageArgs& a, int e0, TC* sR) {
   if (!a.Rsrc) return;
   constexpr int NV = D + 2;
-  for (int idx = threadIdx.x; idx < NB * EPB; idx += kThreads) {
+  for (int idx = threadIdx.x; idx < NB * EPB; idx += NT) {
     const int b = idx / EPB, le = idx % EPB, e = e0 + le;
     if (e < g.E) sR[b * 16 + le * NV + D] += static_cast<TC>(a.Rsrc[static_cast<int64_t>(e) * NB + b]);
   }
@@ -149,6 +159,7 @@ __device__ __forceinline__ void mfmaStageTail(const Geo& g, const StageArgs& a, 
   constexpr int NV = D + 2, NAQ = NF * NFQ;
   constexpr int NBk = r4(NB), NBm = r16(NB), NQm = r16(NQ), NAQm = r16(NAQ);
   constexpr bool MIX = sizeof(TC) == 4;
+  constexpr int STEP = MfmaShape<NB, NQ, NAQ>::STEP, WAVES = MfmaShape<NB, NQ, NAQ>::WAVES;
   const MOpsT<TC>& op = opsOf<TC>(g);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
@@ -158,7 +169,7 @@ __device__ __forceinline__ void mfmaStageTail(const Geo& g, const StageArgs& a, 
   if (a.last_stage) {  // residual monitor: mean_q |R V^T| (TimeIntegration.cpp:279-298)
     double part = 0.0;
     #pragma unroll 1
-    for (int m0 = wave * 16; m0 < NQm; m0 += 64) {
+    for (int m0 = wave * 16; m0 < NQm; m0 += STEP) {
       acc_t<TC> acc = zeroAcc<TC>();
       tileAcc<TC, NQm>(acc, op.rinterp, m0, sR, 0, NBk, lane);
 #pragma unroll
@@ -173,14 +184,16 @@ __device__ __forceinline__ void mfmaStageTail(const Geo& g, const StageArgs& a, 
     if (lane < 16) sRed[wave * 16 + lane] = part;
     __syncthreads();
     if (tid < EPB * NV && e0 + tid / NV < g.E) {
-      const double s = sRed[tid] + sRed[16 + tid] + sRed[32 + tid] + sRed[48 + tid];
+      double s = sRed[tid];
+#pragma unroll
+      for (int w = 1; w < WAVES; w++) s += sRed[16 * w + tid];
       a.mon[static_cast<int64_t>(e0 + tid / NV) * NV + tid % NV] = s / NQ;
     }
   }
   // update: U <- c1 U + c0 Un + c2dt (R Mref^-1) / |J|, in FP64 in both modes; in the mixed mode
   // the FP32 residual panel is mapped to the hierarchic coefficients by FP64 matrix cores
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<double> acc = zeroAcc<double>();
     if constexpr (MIX) {
       const int kr = lane >> 4;
@@ -253,7 +266,7 @@ __device__ __forceinline__ void mfmaStageTail(const Geo& g, const StageArgs& a, 
   // traces of the new state
   TC* Uf_out = pick<TC>(a.Uf_out, a.Uf_out32);
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NAQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NAQm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NAQm>(acc, op.trace, m0, sU, 0, NBk, lane);
 #pragma unroll
@@ -307,12 +320,13 @@ __device__ __forceinline__ void volumeFlux(const StageArgs& a, const double* w, 
 
 // ---- Euler stage (MFMA) -------------------------------------------------------------------------
 template <typename TC, int D, int NB, int NQ, int NF, int NFQ>
-__global__ __launch_bounds__(kThreads) void eulerStageMfma(Geo g, Phys ph, StageArgs a) {
+__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void eulerStageMfma(Geo g, Phys ph, StageArgs a) {
   const MOpsT<TC>& op = opsOf<TC>(g);
   constexpr int NV = D + 2, NAQ = NF * NFQ;
   constexpr int EPB = 16 / NV;
   constexpr int NBk = r4(NB), NBm = r16(NB), NQm = r16(NQ), NAQk = r4(NAQ), NDQk = r4(NQ * D);
   constexpr int NBr = NBk > NBm ? NBk : NBm;
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
   __shared__ TC sU[NBr * 16];
   __shared__ TC sUq[NQm * 16];
   __shared__ TC sF[NDQk * 16];
@@ -323,22 +337,22 @@ __global__ __launch_bounds__(kThreads) void eulerStageMfma(Geo g, Phys ph, Stage
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int e0 = blockIdx.x * EPB;
   const TC* Uf_in = pick<TC>(a.Uf_in, a.Uf_in32);
-  zeroLds(sF, NDQk * 16, tid);
-  zeroLds(sH, NAQk * 16, tid);
-  for (int idx = tid; idx < NBr * 16; idx += kThreads) {
+  zeroLds<NT>(sF, NDQk * 16, tid);
+  zeroLds<NT>(sH, NAQk * 16, tid);
+  for (int idx = tid; idx < NBr * 16; idx += NT) {
     const int b = idx / 16, c = idx % 16, le = c / NV, v = c % NV, e = e0 + le;
     sU[idx] = (b < NB && c < EPB * NV && e < g.E) ? stateOperand<TC>(a, e, v, b, NV, NB) : TC(0);
   }
   __syncthreads();
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NQm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NQm>(acc, op.interp, m0, sU, 0, NBk, lane);
     tileStore<TC>(acc, sUq, m0, lane);
   }
   __syncthreads();
   // volume flux at the points: (F^T (J^T)^-1 |J| w) -> sF[(q D + b)][le NV + v]
-  for (int idx = tid; idx < EPB * NQ; idx += kThreads) {
+  for (int idx = tid; idx < EPB * NQ; idx += NT) {
     const int le = idx / NQ, q = idx % NQ, e = e0 + le;
     if (e >= g.E) continue;
     double u[NV], w[D + 3];
@@ -352,7 +366,7 @@ __global__ __launch_bounds__(kThreads) void eulerStageMfma(Geo g, Phys ph, Stage
       for (int v = 0; v < NV; v++) sF[(q * D + b) * 16 + le * NV + v] = static_cast<TC>(out[b * NV + v]);
   }
   // face fluxes -> sH[slot][le NV + v] (negated: the face term enters the residual with -)
-  for (int idx = tid; idx < EPB * NAQ; idx += kThreads) {
+  for (int idx = tid; idx < EPB * NAQ; idx += NT) {
     const int le = idx / NAQ, sl = idx % NAQ, e = e0 + le;
     if (e >= g.E) continue;
     const int64_t es = static_cast<int64_t>(e) * NAQ + sl;
@@ -393,17 +407,17 @@ __global__ __launch_bounds__(kThreads) void eulerStageMfma(Geo g, Phys ph, Stage
   __syncthreads();
   // residual R = F Phi_grad - H Phi_face
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NBm>(acc, op.grad, m0, sF, 0, NDQk, lane);
     tileAcc<TC, NBm>(acc, op.face, m0, sH, 0, NAQk, lane);
     tileStore<TC>(acc, sR, m0, lane);
   }
-  for (int idx = NBm * 16 + tid; idx < NBr * 16; idx += kThreads) sR[idx] = TC(0);
+  for (int idx = NBm * 16 + tid; idx < NBr * 16; idx += NT) sR[idx] = TC(0);
   __syncthreads();
-  addSource<TC, D, NB, EPB>(g, a, e0, sR);
+  addSource<TC, D, NB, EPB, NT>(g, a, e0, sR);
   if (a.mode == 1) {
-    for (int idx = tid; idx < NB * 16; idx += kThreads) {
+    for (int idx = tid; idx < NB * 16; idx += NT) {
       const int b = idx / 16, c = idx % 16, le = c / NV, v = c % NV, e = e0 + le;
       if (c < EPB * NV && e < g.E) {
         double r = sR[idx];
@@ -447,6 +461,7 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   constexpr int NV = LD::NV, NG = LD::NG, NAQ = LD::NAQ, EPB = LD::EPB;
   constexpr int NBk = LD::NBk, NBm = LD::NBm, NQm = LD::NQm, NAQk = LD::NAQk, NAQm = LD::NAQm, NDQk = LD::NDQk;
   constexpr int NBr = LD::NBr, AJ = LD::AJ;
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
   TC* sU = sRR;
   TC* sA = sAJ;
   TC* sJ = sAJ + NAQk * 16;
@@ -456,14 +471,14 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
   const TC* Uf_in = pick<TC>(a.Uf_in, a.Uf_in32);
-  zeroLds(sAJ, AJ, tid);
-  for (int idx = tid; idx < NBr * 16; idx += kThreads) {
+  zeroLds<NT>(sAJ, AJ, tid);
+  for (int idx = tid; idx < NBr * 16; idx += NT) {
     const int b = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
     sU[idx] = (b < NB && cc < EPB * NV && e < g.E) ? stateOperand<TC>(a, e, v, b, NV, NB) : TC(0);
   }
   __syncthreads();
   // face terms: (u- + u+)/2 (x) n |J_f| w (signed by side) and (u+ - u-)/2 (x) n |J_f| w
-  for (int idx = tid; idx < EPB * NAQ * NV; idx += kThreads) {
+  for (int idx = tid; idx < EPB * NAQ * NV; idx += NT) {
     const int le = idx / (NAQ * NV), rem = idx % (NAQ * NV), sl = rem / NV, v = rem % NV, e = e0 + le;
     if (e >= g.E) continue;
     const int64_t es = static_cast<int64_t>(e) * NAQ + sl;
@@ -493,7 +508,7 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   }
   // state at the volume points
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NQm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NQm>(acc, op.interp, m0, sU, 0, NBk, lane);
     tileStore<TC>(acc, sUq, m0, lane);
@@ -511,7 +526,7 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
 #pragma unroll
     for (int b = 0; b < D; b++) gi[b] = g.ginv[static_cast<int64_t>(gec) * D * D + ga + D * b];
     #pragma unroll 1
-    for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+    for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
       acc_t<TC> aw = zeroAcc<TC>(), aj = zeroAcc<TC>();
       tileAcc<TC, NBm>(aw, op.face, m0, sA, 0, NAQk, lane);
       tileAcc<TC, NBm>(aj, op.face, m0, sJ, 0, NAQk, lane);
@@ -532,13 +547,13 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
       tileStore<TC>(at, sRt, m0, lane);
     }
   }
-  for (int idx = NBm * 16 + tid; idx < NBr * 16; idx += kThreads) sRw[idx] = sRt[idx] = TC(0);
+  for (int idx = NBm * 16 + tid; idx < NBr * 16; idx += NT) sRw[idx] = sRt[idx] = TC(0);
   __syncthreads();
   const double idj = 1.0 / dj;
   // optional output of the lifted total-gradient coefficients w = R_t Mref^-1 / |J|
   if (a.Wout) {
     #pragma unroll 1
-    for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+    for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
       acc_t<TC> wt = zeroAcc<TC>();
       tileAcc<TC, NBm>(wt, op.minv, m0, sRt, 0, NBk, lane);
 #pragma unroll
@@ -551,7 +566,7 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   // lifted gradient traces at the face points -> HBM
   TC* Gf = pick<TC>(a.Gf, a.Gf32);
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NAQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NAQm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     if (VISC == 2) {
       tileAcc<TC, NAQm>(acc, op.ptrace, m0, sRw, 0, NBk, lane);
@@ -574,7 +589,7 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   __syncthreads();
   // total gradient at the volume points (into the face-term buffer, no longer needed)
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NQm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NQm>(acc, op.pinterp, m0, VISC == 0 ? sRw : sRt, 0, NBk, lane);
 #pragma unroll
@@ -585,9 +600,10 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
 }
 
 template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int VISC>
-__global__ __launch_bounds__(kThreads) void nsGradMfma(Geo g, Phys ph, StageArgs a) {
+__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsGradMfma(Geo g, Phys ph, StageArgs a) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
   constexpr int NV = LD::NV, NG = LD::NG, EPB = LD::EPB;
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT;
   __shared__ TC sUq[LD::NQm * 16];      // state at volume points
   __shared__ TC sAJ[LD::AJ];            // face terms A | J ([slot][le*NG + r]); later the gradient at points
   __shared__ TC sRR[2 * LD::NBr * 16];  // state panel; then R_w | R_t
@@ -599,7 +615,7 @@ __global__ __launch_bounds__(kThreads) void nsGradMfma(Geo g, Phys ph, StageArgs
   // volume flux (F_c - F_v)^T (J^T)^-1 |J| w at the points -> HBM Fv[e][(q D + b)][v]; the weak
   // divergence F Phi_grad is taken in nsResidualMfma, which packs three elements per 16 columns
   TC* Fv = pick<TC>(a.Fv, a.Fv32);
-  for (int idx = tid; idx < EPB * NQ; idx += kThreads) {
+  for (int idx = tid; idx < EPB * NQ; idx += NT) {
     const int le = idx / NQ, q = idx % NQ, e = e0 + le;
     if (e >= g.E) continue;
     double u[NV], w[D + 3], gq[NG], pg[NG], fv[D * NV];
@@ -746,13 +762,14 @@ __global__ __launch_bounds__(kThreads) void nsFaceFluxKernel(Geo g, Phys ph, Sta
 // calculateResidual + updateBasisFunctionCoefficient (SpatialDiscrete.cpp:1016-1032,
 // TimeIntegration.cpp:181-198)
 template <typename TC, int D, int NB, int NQ, int NF, int NFQ>
-__global__ __launch_bounds__(kThreads) void nsResidualMfma(Geo g, Phys ph, StageArgs a) {
+__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsResidualMfma(Geo g, Phys ph, StageArgs a) {
   const MOpsT<TC>& op = opsOf<TC>(g);
   constexpr int NV = D + 2, NAQ = NF * NFQ;
   constexpr int EPB = 16 / NV;
   constexpr int NBk = r4(NB), NBm = r16(NB), NAQk = r4(NAQ);
   constexpr int NBr = NBk > NBm ? NBk : NBm;
   constexpr int NDQ = NQ * D, NDQk = r4(NDQ);
+  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
   __shared__ TC sU[NBr * 16];
   __shared__ TC sH[NAQk * 16];
   __shared__ TC sF[NDQk * 16];
@@ -764,31 +781,31 @@ __global__ __launch_bounds__(kThreads) void nsResidualMfma(Geo g, Phys ph, Stage
   const TC* Hs = pick<TC>(static_cast<const double*>(a.Hs), static_cast<const float*>(a.Hs32));
   const TC* Fv = pick<TC>(static_cast<const double*>(a.Fv), static_cast<const float*>(a.Fv32));
   if constexpr (sizeof(TC) == 8) {  // the mixed-precision tail reads the FP64 state from HBM
-    for (int idx = tid; idx < NBr * 16; idx += kThreads) {
+    for (int idx = tid; idx < NBr * 16; idx += NT) {
       const int b = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
       sU[idx] = (b < NB && cc < EPB * NV && e < g.E) ? a.U[(static_cast<int64_t>(e) * NV + v) * NB + b] : 0.0;
     }
   }
-  for (int idx = tid; idx < NAQk * 16; idx += kThreads) {
+  for (int idx = tid; idx < NAQk * 16; idx += NT) {
     const int sl = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
     sH[idx] = (sl < NAQ && cc < EPB * NV && e < g.E) ? Hs[(static_cast<int64_t>(e) * NV + v) * NAQ + sl] : TC(0);
   }
-  for (int idx = tid; idx < NDQk * 16; idx += kThreads) {
+  for (int idx = tid; idx < NDQk * 16; idx += NT) {
     const int k = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
     sF[idx] = (k < NDQ && cc < EPB * NV && e < g.E) ? Fv[(static_cast<int64_t>(e) * NDQ + k) * NV + v] : TC(0);
   }
   __syncthreads();
   #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NBm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NBm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NBm>(acc, op.grad, m0, sF, 0, NDQk, lane);
     tileAcc<TC, NBm>(acc, op.face, m0, sH, 0, NAQk, lane);
     tileStore<TC>(acc, sR, m0, lane);
   }
   __syncthreads();
-  addSource<TC, D, NB, EPB>(g, a, e0, sR);
+  addSource<TC, D, NB, EPB, NT>(g, a, e0, sR);
   if (a.mode == 1) {
-    for (int idx = tid; idx < NB * 16; idx += kThreads) {
+    for (int idx = tid; idx < NB * 16; idx += NT) {
       const int b = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
       if (cc < EPB * NV && e < g.E) {
         double r = sR[idx];
@@ -805,15 +822,16 @@ __global__ __launch_bounds__(kThreads) void nsResidualMfma(Geo g, Phys ph, Stage
 // matrix-core accumulation order as the stage tail that produces them after every stage, so a state
 // set from the host (a restart, a checkpoint) continues bit-identically. EPB elements per block.
 template <typename TC, int D, int NB, int NF, int NFQ>
-__global__ __launch_bounds__(kThreads) void mfmaTraceKernel(Geo g, const double* U, void* Uf_out, MixRef mix) {
+__global__ __launch_bounds__((MfmaShape<NB, NB, NF * NFQ>::NT)) void mfmaTraceKernel(Geo g, const double* U, void* Uf_out, MixRef mix) {
   constexpr int NV = D + 2, NAQ = NF * NFQ, EPB = 16 / NV;
   constexpr int NBk = r4(NB), NAQm = r16(NAQ);
+  constexpr int NT = MfmaShape<NB, NB, NAQ>::NT, STEP = MfmaShape<NB, NB, NAQ>::STEP;
   __shared__ TC sU[NBk * 16];
   const MOpsT<TC>& op = opsOf<TC>(g);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
   const int e0 = blockIdx.x * EPB;
-  for (int idx = tid; idx < NBk * 16; idx += kThreads) {
+  for (int idx = tid; idx < NBk * 16; idx += NT) {
     const int b = idx / 16, cc = idx % 16, le = cc / NV, v = cc % NV, e = e0 + le;
     TC x = TC(0);
     if (b < NB && cc < EPB * NV && e < g.E) {
@@ -830,7 +848,7 @@ __global__ __launch_bounds__(kThreads) void mfmaTraceKernel(Geo g, const double*
   const bool col_ok = c < EPB * NV && e < g.E;
   TC* out = static_cast<TC*>(Uf_out);
 #pragma unroll 1
-  for (int m0 = wave * 16; m0 < NAQm; m0 += 64) {
+  for (int m0 = wave * 16; m0 < NAQm; m0 += STEP) {
     acc_t<TC> acc = zeroAcc<TC>();
     tileAcc<TC, NAQm>(acc, op.trace, m0, sU, 0, NBk, lane);
 #pragma unroll

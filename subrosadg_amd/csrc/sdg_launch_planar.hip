@@ -1,0 +1,29 @@
+// sdg_launch_planar.hip -- kernel sets of lines and triangles
+#include "launchers.hpp"
+
+namespace sdg {
+
+// 1-D: vector kernels (P+1 modes, P+1 Gauss points, two end-point faces)
+bool selectLine(int order, bool mixed, Launchers& l) {
+  switch (order) {
+    case 1: return pickValu<1, 2, 2, 2, 1>(mixed, l);
+    case 2: return pickValu<1, 3, 3, 2, 1>(mixed, l);
+    case 3: return pickValu<1, 4, 4, 2, 1>(mixed, l);
+    case 4: return pickValu<1, 5, 5, 2, 1>(mixed, l);
+    case 5: return pickValu<1, 6, 6, 2, 1>(mixed, l);
+    default: return false;
+  }
+}
+
+// bases of 3..15 functions: vector kernels
+bool selectTriangle(int order, bool mixed, Launchers& l) {
+  switch (order) {
+    case 1: return pickValu<2, 3, 3, 3, 2>(mixed, l);
+    case 2: return pickValu<2, 6, 6, 3, 3>(mixed, l);
+    case 3: return pickValu<2, 10, 12, 3, 4>(mixed, l);
+    case 4: return pickValu<2, 15, 16, 3, 5>(mixed, l);
+    default: return false;
+  }
+}
+
+}  // namespace sdg

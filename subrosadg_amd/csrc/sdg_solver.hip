@@ -72,7 +72,7 @@ inline int blocksFor(int E, int epb) { return (E + epb - 1) / epb; }
 
 // VALU kernels: any size; MFMA kernels: bases that fill 16x16 tiles. TC is the contraction type of
 // the matrix-core kernels: double (FP64 mode) or float (mixed-precision mode).
-template <int D, int NB, int NQ, int NF, int NFQ, bool MFMA, typename TC = double>
+template <int D, int NB, int NQ, int NF, int NFQ, bool MFMA, typename TC = double, bool ADJOINT = true>
 Launchers makeLaunchers() {
   using S = sdg::Sizes<D, NB, NQ, NF, NFQ>;
   constexpr int EPB = S::EPB;
@@ -83,14 +83,14 @@ Launchers makeLaunchers() {
     constexpr int EPB_S = 16 / NV, EPB_G = 16 / (NV * D);
     l.euler = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
       hipLaunchKernelGGL((sdg::eulerStageMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
+                         dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
     };
     l.ns_grad_br1 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)), dim3(sdg::kThreads),
+      hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)), dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT),
                          0, st, g, ph, a);
     };
     l.ns_grad_br2 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)), dim3(sdg::kThreads),
+      hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)), dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT),
                          0, st, g, ph, a);
     };
     l.ns_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
@@ -98,33 +98,33 @@ Launchers makeLaunchers() {
                          dim3(sdg::kThreads), 0, st, g, ph, a);
     };
     l.ns_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)), dim3(sdg::kThreads),
+      hipLaunchKernelGGL((sdg::nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)), dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT),
                          0, st, g, ph, a);
     };
     {  // Euler with artificial viscosity: volume gradient, AV fluxes (both precision modes)
       l.av_grad = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
         hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 0>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
       };
       l.av_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
         hipLaunchKernelGGL((sdg::nsFaceFluxKernel<TC, D, NF, NFQ, false, true>),
                            dim3(blocksFor((g.F + g.Fb) * NFQ, sdg::kThreads)), dim3(sdg::kThreads), 0, st, g, ph, a);
         hipLaunchKernelGGL((sdg::nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
       };
       l.av_sensor = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, double* node) {
         hipLaunchKernelGGL((sdg::avSensorKernel<D, NB, NQ>), dim3(blocksFor(g.E, sdg::kThreads)), dim3(sdg::kThreads),
                            0, st, g, ph, U, node);
       };
     }
-    if constexpr (sizeof(TC) == 8) {
+    if constexpr (ADJOINT && sizeof(TC) == 8) {
       l.adj_volume[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
         hipLaunchKernelGGL((sdg::nsAdjVolumeMfma<D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a, j);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_volume[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
         hipLaunchKernelGGL((sdg::nsAdjVolumeMfma<D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a, j);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
         if (ph.flux <= SDG_FLUX_ROE)  // reverse mode, one thread per face point
@@ -137,15 +137,15 @@ Launchers makeLaunchers() {
       };
       l.adj_lift[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
         hipLaunchKernelGGL((sdg::nsAdjLiftMfma<D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a, j);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_lift[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
         hipLaunchKernelGGL((sdg::nsAdjLiftMfma<D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a, j);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_gather = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
         hipLaunchKernelGGL((sdg::nsAdjGatherMfma<D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                           dim3(sdg::kThreads), 0, st, g, ph, a, j);
+                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
     }
   } else {
@@ -194,7 +194,7 @@ Launchers makeLaunchers() {
     // the stage tail's own contraction (bit-identical traces after a host-side state change)
     l.trace = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const sdg::MixRef& mix) {
       hipLaunchKernelGGL((sdg::mfmaTraceKernel<TC, D, NB, NF, NFQ>), dim3(blocksFor(g.E, 16 / (D + 2))),
-                         dim3(sdg::kThreads), 0, st, g, U, Uf, mix);
+                         dim3(sdg::MfmaShape<NB, NB, NF * NFQ>::NT), 0, st, g, U, Uf, mix);
     };
   } else {
     l.trace = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const sdg::MixRef& mix) {
@@ -234,6 +234,13 @@ bool pickMfma(bool force_valu, bool mixed, Launchers& l) {
     l = makeLaunchers<D, NB, NQ, NF, NFQ, true, float>();
   else
     l = force_valu ? makeLaunchers<D, NB, NQ, NF, NFQ, false>() : makeLaunchers<D, NB, NQ, NF, NFQ, true>();
+  return true;
+}
+// Tetrahedra: the FP64 matrix-core kernels, without the mixed mode and the adjoint of pickMfma
+template <int NB, int NQ, int NFQ>
+bool pickTet(bool force_valu, bool mixed, Launchers& l) {
+  if (mixed) return false;
+  l = force_valu ? makeLaunchers<3, NB, NQ, 4, NFQ, false>() : makeLaunchers<3, NB, NQ, 4, NFQ, true, double, false>();
   return true;
 }
 template <int D, int NB, int NQ, int NF, int NFQ>
@@ -378,12 +385,12 @@ bool selectLaunchers(int type, int order, bool force_valu, bool mixed, Launchers
       default: return false;
     }
   }
-  if (type == SDG_ELEM_TETRAHEDRON) {  // bases of 4..35 functions, Grundmann-Moeller volume rules: vector kernels
+  if (type == SDG_ELEM_TETRAHEDRON) {  // bases of 4..35 functions, Grundmann-Moeller volume rules
     switch (order) {
-      case 1: return pickValu<3, 4, 5, 4, 4>(mixed, l);
-      case 2: return pickValu<3, 10, 15, 4, 7>(mixed, l);
-      case 3: return pickValu<3, 20, 35, 4, 13>(mixed, l);
-      case 4: return pickValu<3, 35, 70, 4, 19>(mixed, l);
+      case 1: return pickTet<4, 5, 4>(force_valu, mixed, l);
+      case 2: return pickTet<10, 15, 7>(force_valu, mixed, l);
+      case 3: return pickTet<20, 35, 13>(force_valu, mixed, l);
+      case 4: return pickTet<35, 70, 19>(force_valu, mixed, l);
       default: return false;
     }
   }
