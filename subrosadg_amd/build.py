@@ -19,7 +19,8 @@ BUILD_DIR = os.path.join(HERE, "_build")
 HOST_SOURCES = ["kit.cpp", "sdg_mesh_api.cpp", "sdg_raw.cpp", "sdg_vtu.cpp", "sdg_gmsh.cpp"]
 # the system zstd runtime (raw state files); only its stable C API is used
 LINK_LIBS = ["-l:libzstd.so.1"]
-HIP_SOURCES = ["sdg_solver.hip", "sdg_batch.hip"]
+HIP_SOURCES = ["sdg_solver.hip", "sdg_batch.hip"] + [f"sdg_launch_{k}.hip" for k in
+                                                       ("planar", "quad", "pyramid", "tet", "hex", "tensor")]
 EXAMPLES = ["taylor_green_3d_cns", "lid_driven_cavity_2d_cns", "shear_layer_2d_cns_restart", "thermal_cavity_3d_cns",
             "explosion_2d_ceuler", "mesh_file_2d_ceuler", "sod_1d_ceuler",
             "pulsed_inflow_2d_ceuler"]

@@ -163,8 +163,9 @@ struct MixRef {
 };
 
 struct StageArgs {
-  double* U;
-  double* Un;
+  const double* U;   // state the stage evaluates
+  const double* Un;  // state at the start of the step
+  double* Uo;        // updated state (may be U or Un: an entry is read before its own thread writes it)
   const double* Uf_in;
   double* Uf_out;
   double* Gf;
@@ -334,11 +335,10 @@ __device__ __forceinline__ void stageTail(const Geo& g, const StageArgs& a, int 
     }
     const int64_t gi = static_cast<int64_t>(e) * NV * NB + rem;
     double u = sU[le][v][i] * a.c1;
-    u += a.c0 * a.Un[gi];
+    if (a.c0 != 0.0) u += a.c0 * a.Un[gi];
     u += a.c2dt * rm;
     sU[le][v][i] = u;
-    a.U[gi] = u;
-    if (a.last_stage) a.Un[gi] = u;
+    a.Uo[gi] = u;
   }
   __syncthreads();
   // traces of the new state for the next stage
@@ -945,7 +945,7 @@ __global__ __launch_bounds__(kThreads) void nsFluxKernel(Geo g, Phys ph, StageAr
 }
 
 // ---- artificial viscosity (SpatialDiscrete.cpp:37-192) ----------------------------------------
-__global__ __launch_bounds__(kThreads) void avClearKernel(double* node, int64_t n) {
+inline __global__ __launch_bounds__(kThreads) void avClearKernel(double* node, int64_t n) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * kThreads)
     node[i] = 0.0;
@@ -1156,7 +1156,7 @@ __global__ __launch_bounds__(kThreads) void monitorKernel(const double* part, in
   }
 }
 
-__global__ void resetStatusKernel(int* status) {
+inline __global__ void resetStatusKernel(int* status) {
   if (threadIdx.x == 0) {
     status[0] = 0;
     status[1] = 0;

@@ -682,7 +682,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsResidualTensor(Geo g, P
     const int b = t.iperm[q];
     for (int v = 0; v < NV; v++) {
       pu[v] = a.U[(e * NV + v) * NPT + b];
-      pn[v] = a.Un[(e * NV + v) * NPT + b];
+      pn[v] = a.c0 != 0.0 ? a.Un[(e * NV + v) * NPT + b] : 0.0;
     }
     // compile-time trip counts, so that all the loads are issued before the first wait
 #pragma unroll  // the weak divergence of the volume flux at the node (gradient kernel)
@@ -782,8 +782,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsResidualTensor(Geo g, P
       double u = pu[v] * a.c1;
       u += a.c0 * pn[v];
       u += a.c2dt * T0[v * NPT + q];
-      a.U[gi] = u;
-      if (a.last_stage) a.Un[gi] = u;
+      a.Uo[gi] = u;
       if (a.rec) {
         const int step = a.status[1] + (a.last_stage ? 1 : 0);
         const int stage = a.last_stage ? 0 : a.rec_stage + 1;

@@ -207,8 +207,8 @@ Launchers makeLaunchers() {
   l.monitor = [](hipStream_t st, const double* mon, int E, double* rel, int* status) {
     // mon holds E x NV per-element values followed by kMonitorBlocks x NV partial sums
     double* part = const_cast<double*>(mon) + static_cast<int64_t>(E) * (D + 2);
-    hipLaunchKernelGGL((monitorKernel<D + 2>), dim3(monitorBlocks(E, D + 2)), dim3(kThreads), 0, st, mon, E, part, rel,
-                       status);
+    hipLaunchKernelGGL((monitorPartialKernel<D + 2>), dim3(kMonitorBlocks), dim3(kThreads), 0, st, mon, E, part, status);
+    hipLaunchKernelGGL((monitorKernel<D + 2>), dim3(1), dim3(kThreads), 0, st, part, E, rel, status);
   };
   return l;
 }
@@ -321,7 +321,8 @@ bool selectTensorAvT(int order, Launchers& l) {
   }
 }
 // Quadrangles, FP64: the sum-factorised stage kernels replace those of every stage (the adjoint kernels
-// stay). 256^2 P3 Euler + AV: 98 us of kernels a stage against 260 us on the matrix-core kernels.
+// stay). 256^2 P3 Euler with artificial viscosity: 95 us of kernels a stage, 260 us on the matrix-core
+// kernels; 48^2 P3 Navier-Stokes: 14.3 us and 28 us; 32^2 P2 Euler: 7.1 us and 8.5 us on the vector kernel.
 template <int N>
 bool pickQuad(Launchers& l) {
   constexpr int EPB = QuadShape<N>::EPB;

@@ -65,8 +65,9 @@ struct WorkItem {
 // element is the face's right parent, bit 1 the neighbour's points run in reverse order.
 template <typename TC>
 struct Args {
-  double* U;
-  double* Un;
+  const double* U;   // state the stage evaluates
+  const double* Un;  // state at the start of the step
+  double* Uo;        // updated state (may be U or Un: an entry is read before its own thread writes it)
   const TC* Tin;
   TC* Tout;
   const double* ginv;   // per element: (J^T)^-1 column-major 2 x 2
@@ -82,7 +83,6 @@ struct Args {
   const VariantDev* var;
   const WorkItem* items;
   int nitems;
-  int last_stage;
   double c0, c1, c2;
   Phys ph;
 };
@@ -150,7 +150,7 @@ __device__ __forceinline__ TC traceAt(const TC* su, const TC* tVft, int sl) {
 //   A      one thread per volume point: point values (FP32 / FP64 contraction), FP64 flux
 //          F^T (J^T)^-1 |J| w; one thread per face slot: the own trace from the panel, the
 //          neighbour's from HBM, the numerical flux with the face's left/right roles
-//   B      one thread per mode: R = F . grad psi - H psi, RK update in FP64 (U, U_n), new state
+//   B      one thread per mode: R = F . grad psi - H psi, RK update in FP64, new state
 //          operand into the panel
 //   C      traces of the new state for the neighbours (slot-major, the variables of a slot adjacent)
 template <typename TC, int FLUX, int NB, int NQ, int NF, int NFQ>
@@ -336,8 +336,7 @@ __device__ __forceinline__ void eulerTile(const Args<TC>& a, const VariantDev& v
         double u = uo[v] * a.c1;
         u += a.c0 * uno[v];
         u += scale * rm[v];
-        a.U[gi] = u;
-        if (a.last_stage) a.Un[gi] = u;
+        a.Uo[gi] = u;
         sU[le][v][i] = stateOperand<TC>(u, MIX ? a.mix[p * 6 + v] : 0.0, onei);
       }
     }
@@ -481,7 +480,7 @@ __global__ __launch_bounds__(kThreads) void batchToReferenceKernel(const double*
   for (int v = 0; v < NV; v++) o[v] = acc[v];
 }
 __global__ __launch_bounds__(kThreads) void batchFromReferenceKernel(const double* in, const int64_t* coff, int64_t n,
-                                                                     int nb, const double* Lc, double* U, double* Un) {
+                                                                     int nb, const double* Lc, double* U) {
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (idx >= n * nb) return;
   const int64_t e = idx / nb;
@@ -492,10 +491,7 @@ __global__ __launch_bounds__(kThreads) void batchFromReferenceKernel(const doubl
     const double l = Lc[i * nb + j];
     for (int v = 0; v < NV; v++) acc[v] += l * c[i * NV + v];
   }
-  for (int v = 0; v < NV; v++) {
-    U[(e * NV + v) * nb + j] = acc[v];
-    Un[(e * NV + v) * nb + j] = acc[v];
-  }
+  for (int v = 0; v < NV; v++) U[(e * NV + v) * nb + j] = acc[v];
 }
 
 }  // namespace batch
@@ -519,7 +515,7 @@ struct sdg_batch {
   std::vector<std::vector<std::pair<int, int64_t>>> emap;  // problem, element -> (variant, index)
   std::vector<std::vector<int64_t>> coeff_off;             // problem, element -> offset in reference layout
   int64_t totalE = 0, totalU = 0, totalT = 0, totalF = 0;
-  double *U = nullptr, *Un = nullptr, *ginv = nullptr, *detj = nullptr, *fnrm = nullptr, *fjw = nullptr, *dt = nullptr,
+  double *U = nullptr, *Us = nullptr, *ginv = nullptr, *detj = nullptr, *fnrm = nullptr, *fjw = nullptr, *dt = nullptr,
          *mix = nullptr, *min_edge = nullptr, *dtbuf = nullptr;
   int* pid = nullptr;
   int64_t* fnb = nullptr;
@@ -597,7 +593,8 @@ template <typename TC>
 Args<TC> makeArgs(sdg_batch* b, int parity) {
   Args<TC> a{};
   a.U = b->U;
-  a.Un = b->Un;
+  a.Un = b->U;
+  a.Uo = b->U;
   a.Tin = static_cast<const TC*>(b->T[parity]);
   a.Tout = static_cast<TC*>(b->T[parity ^ 1]);
   a.ginv = b->ginv;
@@ -679,7 +676,9 @@ void launchStageT(sdg_batch* b, int stage, int parity, int only) {
   a.c0 = c[0];
   a.c1 = c[1];
   a.c2 = c[2];
-  a.last_stage = stage == stagesOf(b) - 1;
+  // the step-start state stays in U until the last stage replaces it; the stages between work in Us
+  if (stage > 0) a.U = b->Us;
+  if (stage < stagesOf(b) - 1) a.Uo = b->Us;
   if (only >= 0) {
     launchVariant<TC>(b, a, only, b->stream);
     return;
@@ -995,7 +994,7 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
       bupload(b, pid, &b->pid) || bupload(b, coff, &b->coff) ||
       balloc(b, static_cast<size_t>(*std::max_element(b->ncoeff.begin(), b->ncoeff.end())), &b->io) || bupload(b, fnb, &b->fnb) || bupload(b, fid, &b->fid) || bupload(b, fflag, &b->fflag) ||
       bupload(b, fnrm, &b->fnrm) || bupload(b, fjw, &b->fjw) || balloc(b, static_cast<size_t>(ub), &b->U) ||
-      balloc(b, static_cast<size_t>(ub), &b->Un) || balloc(b, static_cast<size_t>(count), &b->dt) ||
+      balloc(b, static_cast<size_t>(ub), &b->Us) || balloc(b, static_cast<size_t>(count), &b->dt) ||
       balloc(b, static_cast<size_t>(count) * 6, &b->mix) || balloc(b, static_cast<size_t>(eb), &b->dtbuf) ||
       balloc(b, static_cast<size_t>(tb) * tbytes, reinterpret_cast<char**>(&t0)) ||
       balloc(b, static_cast<size_t>(tb) * tbytes, reinterpret_cast<char**>(&t1)))
@@ -1045,11 +1044,10 @@ int sdg_batch_set_state(sdg_batch* b, int p, const double* coeff) {
     const auto [lo, n] = b->range[p][v];
     if (n == 0) continue;
     const auto& V = b->var[v];
-    const int64_t off = V.u_base + lo * 4 * V.nb;
     hipLaunchKernelGGL(sdg::batch::batchFromReferenceKernel,
                        dim3(static_cast<unsigned>((n * V.nb + sdg::batch::kThreads - 1) / sdg::batch::kThreads)),
                        dim3(sdg::batch::kThreads), 0, b->stream, b->io, b->coff + V.e_base + lo, n, V.nb, b->chol[v],
-                       b->U + off, b->Un + off);
+                       b->U + V.u_base + lo * 4 * V.nb);
   }
   BHIP(b, hipGetLastError());
   BHIP(b, hipMemcpyAsync(b->mix + static_cast<size_t>(p) * 6, &b->mixh[static_cast<size_t>(p) * 6], 6 * sizeof(double),
@@ -1186,9 +1184,9 @@ int sdg_batch_tune(sdg_batch* b, double* stage_ms) {
   for (int p = 0; p < b->nprob; p++)
     if (!b->has_state[p]) return bfail(b, SDG_E_STATE, "sdg_batch_tune: a problem has no state");
   const size_t tbytes = (b->mixed ? sizeof(float) : sizeof(double)) * static_cast<size_t>(b->totalT);
-  std::vector<char> saveU(static_cast<size_t>(b->totalU) * sizeof(double)), saveUn(saveU.size()), saveT(tbytes);
+  std::vector<char> saveU(static_cast<size_t>(b->totalU) * sizeof(double)), saveUs(saveU.size()), saveT(tbytes);
   BHIP(b, hipMemcpy(saveU.data(), b->U, saveU.size(), hipMemcpyDeviceToHost));
-  BHIP(b, hipMemcpy(saveUn.data(), b->Un, saveUn.size(), hipMemcpyDeviceToHost));
+  BHIP(b, hipMemcpy(saveUs.data(), b->Us, saveUs.size(), hipMemcpyDeviceToHost));
   BHIP(b, hipMemcpy(saveT.data(), b->T[b->cur], tbytes, hipMemcpyDeviceToHost));
   auto timeStage = [&](int reps, int only) -> float {
     float best = 1e30f;
@@ -1231,7 +1229,7 @@ int sdg_batch_tune(sdg_batch* b, double* stage_ms) {
   const float best = timeStage(3, -1);
   BHIP(b, hipGetLastError());
   BHIP(b, hipMemcpy(b->U, saveU.data(), saveU.size(), hipMemcpyHostToDevice));
-  BHIP(b, hipMemcpy(b->Un, saveUn.data(), saveUn.size(), hipMemcpyHostToDevice));
+  BHIP(b, hipMemcpy(b->Us, saveUs.data(), saveUs.size(), hipMemcpyHostToDevice));
   BHIP(b, hipMemcpy(b->T[b->cur], saveT.data(), tbytes, hipMemcpyHostToDevice));
   for (int i = 0; i < 2; i++) {
     if (b->graph[i]) (void)hipGraphExecDestroy(b->graph[i]);

@@ -16,410 +16,41 @@
 #include <vector>
 
 #include "../../include/sdg.h"
-#include "dg_adjoint.hpp"
-#include "dg_tensor_adjoint.hpp"
-#include "dg_tensor.hpp"
-#include "dg_kernels.hpp"
-#include "dg_mfma.hpp"
 #include "kit.hpp"
+#include "launchers.hpp"
 #include "sdg_internal.hpp"
 
 using sdg::Geo;
 using sdg::Phys;
 using sdg::StageArgs;
+using sdg::Launchers;
+using sdg::blocksFor;
 
 namespace {
 
-using StageFn = void (*)(hipStream_t, const Geo&, const Phys&, const StageArgs&);
-using TraceFn = void (*)(hipStream_t, const Geo&, const double*, void*, const sdg::MixRef&);
-using DtFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, const double*, double, int, double*);
-using MonFn = void (*)(hipStream_t, const double*, int, double*, int*);
-using SrcFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, double*, const double*);
-using AdjFn = void (*)(hipStream_t, const Geo&, const Phys&, const StageArgs&, const sdg::AdjArgs&);
-using AvFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, double*);
-using BlockFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, double*);
-
-struct Launchers {
-  bool mfma = false;
-  bool tensor = false;  // hexahedra, Navier-Stokes: sum-factorised stage kernels
-  StageFn euler = nullptr;
-  StageFn ns_grad_br1 = nullptr;
-  StageFn ns_grad_br2 = nullptr;
-  StageFn ns_flux = nullptr;
-  StageFn ns_face = nullptr;  // matrix-core path: face fluxes before ns_flux
-  TraceFn trace = nullptr;
-  TraceFn trace64 = nullptr;  // FP64 traces of the FP64 state (the adjoint of mixed-precision contexts)
-  SrcFn source = nullptr;  // modal Boussinesq source (all kernel sets but the sum-factorised one)
-  DtFn dt = nullptr;
-  MonFn monitor = nullptr;
-  // Euler with artificial viscosity (vector kernels): gradient pass + volume flux, face fluxes +
-  // residual + update, and the per-step sensor
-  StageFn av_grad = nullptr;
-  StageFn av_flux = nullptr;
-  StageFn av_ns_grad[2] = {nullptr, nullptr};  // Navier-Stokes with artificial viscosity: BR1, BR2
-  StageFn av_ns_flux = nullptr;
-  AvFn av_sensor = nullptr;
-  // Navier-Stokes BR2 raw files: per boundary face the parent's volume gradient plus that face's lift
-  BlockFn br2_blocks = nullptr;
-  // discrete adjoint (Navier-Stokes, FP64: the dense matrix-core set, or the sum-factorised set on hexahedra)
-  AdjFn adj_volume[2] = {nullptr, nullptr};  // BR1, BR2
-  AdjFn adj_face = nullptr;
-  AdjFn adj_lift[2] = {nullptr, nullptr};
-  AdjFn adj_gather = nullptr;
-};
-
-inline int blocksFor(int E, int epb) { return (E + epb - 1) / epb; }
-
-// VALU kernels: any size; MFMA kernels: bases that fill 16x16 tiles. TC is the contraction type of
-// the matrix-core kernels: double (FP64 mode) or float (mixed-precision mode).
-template <int D, int NB, int NQ, int NF, int NFQ, bool MFMA, typename TC = double, bool ADJOINT = true>
-Launchers makeLaunchers() {
-  using S = sdg::Sizes<D, NB, NQ, NF, NFQ>;
-  constexpr int EPB = S::EPB;
-  constexpr int NV = D + 2;
-  Launchers l;
-  l.mfma = MFMA;
-  if constexpr (MFMA) {
-    constexpr int EPB_S = 16 / NV, EPB_G = 16 / (NV * D);
-    l.euler = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::eulerStageMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                         dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
-    };
-    l.ns_grad_br1 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)), dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT),
-                         0, st, g, ph, a);
-    };
-    l.ns_grad_br2 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)), dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT),
-                         0, st, g, ph, a);
-    };
-    l.ns_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsFaceFluxKernel<TC, D, NF, NFQ>), dim3(blocksFor((g.F + g.Fb) * NFQ, sdg::kThreads)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.ns_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)), dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT),
-                         0, st, g, ph, a);
-    };
-    {  // Euler with artificial viscosity: volume gradient, AV fluxes (both precision modes)
-      l.av_grad = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-        hipLaunchKernelGGL((sdg::nsGradMfma<TC, D, NB, NQ, NF, NFQ, 0>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
-      };
-      l.av_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-        hipLaunchKernelGGL((sdg::nsFaceFluxKernel<TC, D, NF, NFQ, false, true>),
-                           dim3(blocksFor((g.F + g.Fb) * NFQ, sdg::kThreads)), dim3(sdg::kThreads), 0, st, g, ph, a);
-        hipLaunchKernelGGL((sdg::nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
-      };
-      l.av_sensor = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, double* node) {
-        hipLaunchKernelGGL((sdg::avSensorKernel<D, NB, NQ>), dim3(blocksFor(g.E, sdg::kThreads)), dim3(sdg::kThreads),
-                           0, st, g, ph, U, node);
-      };
-    }
-    if constexpr (ADJOINT && sizeof(TC) == 8) {
-      l.adj_volume[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-        hipLaunchKernelGGL((sdg::nsAdjVolumeMfma<D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
-      };
-      l.adj_volume[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-        hipLaunchKernelGGL((sdg::nsAdjVolumeMfma<D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
-      };
-      l.adj_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-        if (ph.flux <= SDG_FLUX_ROE)  // reverse mode, one thread per face point
-          hipLaunchKernelGGL((sdg::nsAdjFaceRevKernel<D, NF, NFQ>), dim3(blocksFor(g.F * NFQ, sdg::kThreads)),
-                             dim3(sdg::kThreads), 0, st, g, ph, a, j);
-        else  // dual numbers, one thread per (state component or gradient, side, face point)
-          hipLaunchKernelGGL((sdg::nsAdjFaceKernel<D, NF, NFQ>),
-                             dim3(blocksFor(g.F * NFQ * 2 * (D + 3), sdg::kThreads)),
-                             dim3(sdg::kThreads), 0, st, g, ph, a, j);
-      };
-      l.adj_lift[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-        hipLaunchKernelGGL((sdg::nsAdjLiftMfma<D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
-      };
-      l.adj_lift[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-        hipLaunchKernelGGL((sdg::nsAdjLiftMfma<D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
-      };
-      l.adj_gather = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-        hipLaunchKernelGGL((sdg::nsAdjGatherMfma<D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                           dim3(sdg::MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
-      };
-    }
-  } else {
-    l.euler = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::eulerStageKernel<D, NB, NQ, NF, NFQ, EPB>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.ns_grad_br1 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradKernel<D, NB, NQ, NF, NFQ, EPB, 1>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.ns_grad_br2 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradKernel<D, NB, NQ, NF, NFQ, EPB, 2>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.ns_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsFluxKernel<D, NB, NQ, NF, NFQ, EPB>), dim3(blocksFor(g.E, EPB)), dim3(sdg::kThreads),
-                         0, st, g, ph, a);
-    };
-    l.av_grad = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradKernel<D, NB, NQ, NF, NFQ, EPB, 0>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.av_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsFluxKernel<D, NB, NQ, NF, NFQ, EPB, 1>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.av_ns_grad[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradKernel<D, NB, NQ, NF, NFQ, EPB, 1, true>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.av_ns_grad[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsGradKernel<D, NB, NQ, NF, NFQ, EPB, 2, true>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.av_ns_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((sdg::nsFluxKernel<D, NB, NQ, NF, NFQ, EPB, 2>), dim3(blocksFor(g.E, EPB)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a);
-    };
-    l.av_sensor = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, double* node) {
-      hipLaunchKernelGGL((sdg::avSensorKernel<D, NB, NQ>), dim3(blocksFor(g.E, sdg::kThreads)), dim3(sdg::kThreads), 0,
-                         st, g, ph, U, node);
-    };
-  }
-  if constexpr (MFMA) {
-    // the stage tail's own contraction (bit-identical traces after a host-side state change)
-    l.trace = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const sdg::MixRef& mix) {
-      hipLaunchKernelGGL((sdg::mfmaTraceKernel<TC, D, NB, NF, NFQ>), dim3(blocksFor(g.E, 16 / (D + 2))),
-                         dim3(sdg::MfmaShape<NB, NB, NF * NFQ>::NT), 0, st, g, U, Uf, mix);
-    };
-  } else {
-    l.trace = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const sdg::MixRef& mix) {
-      const int64_t n = static_cast<int64_t>(g.E) * (D + 2) * NF * NFQ;
-      hipLaunchKernelGGL((sdg::traceKernel<D, NB, NQ, NF, NFQ>), dim3((n + sdg::kThreads - 1) / sdg::kThreads),
-                         dim3(sdg::kThreads), 0, st, g, U, Uf, mix);
-    };
-  }
-  l.source = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, double* out, const double* Li) {
-    constexpr int NM = NQ > NB ? NQ : NB, EPBS = sdg::kThreads / NM > 0 ? sdg::kThreads / NM : 1;
-    hipLaunchKernelGGL((sdg::sourceKernel<D, NB, NQ>), dim3(blocksFor(g.E, EPBS)), dim3(sdg::kThreads), 0, st, g, ph,
-                       U, out, Li);
-  };
-  l.br2_blocks = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, double* out) {
-    hipLaunchKernelGGL((sdg::br2BoundaryBlockKernel<D, NB, NQ, NF, NFQ>), dim3(g.Fb), dim3(sdg::kThreads), 0, st, g, ph,
-                       U, out);
-  };
-  l.dt = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, const double* me, double cfl, int order,
-            double* out) {
-    hipLaunchKernelGGL((sdg::dtKernel<D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, sdg::DtShape<D, NB, NQ>::EPB)),
-                       dim3(sdg::kThreads), 0, st, g, ph, U, me, cfl, order, out);
-  };
-  l.monitor = [](hipStream_t st, const double* mon, int E, double* rel, int* status) {
-    // mon holds E x NV per-element values followed by kMonitorBlocks x NV partial sums
-    double* part = const_cast<double*>(mon) + static_cast<int64_t>(E) * (D + 2);
-    hipLaunchKernelGGL((sdg::monitorPartialKernel<D + 2>), dim3(sdg::kMonitorBlocks), dim3(sdg::kThreads), 0, st, mon,
-                       E, part, status);
-    hipLaunchKernelGGL((sdg::monitorKernel<D + 2>), dim3(1), dim3(sdg::kThreads), 0, st, part, E, rel, status);
-  };
-  return l;
-}
-
-// Kernel set for (element type, order). Mixed precision runs on the matrix-core kernels only.
-template <int D, int NB, int NQ, int NF, int NFQ>
-bool pickMfma(bool force_valu, bool mixed, Launchers& l) {
-  if (mixed)
-    l = makeLaunchers<D, NB, NQ, NF, NFQ, true, float>();
-  else
-    l = force_valu ? makeLaunchers<D, NB, NQ, NF, NFQ, false>() : makeLaunchers<D, NB, NQ, NF, NFQ, true>();
-  return true;
-}
-// Tetrahedra: the FP64 matrix-core kernels, without the mixed mode and the adjoint of pickMfma
-template <int NB, int NQ, int NFQ>
-bool pickTet(bool force_valu, bool mixed, Launchers& l) {
-  if (mixed) return false;
-  l = force_valu ? makeLaunchers<3, NB, NQ, 4, NFQ, false>() : makeLaunchers<3, NB, NQ, 4, NFQ, true, double, false>();
-  return true;
-}
-template <int D, int NB, int NQ, int NF, int NFQ>
-bool pickValu(bool mixed, Launchers& l) {
-  if (mixed) return false;
-  l = makeLaunchers<D, NB, NQ, NF, NFQ, false>();
-  return true;
-}
-
-// Navier-Stokes on hexahedra P2..P4: the sum-factorised stage kernels replace the matrix-core
-// gradient and residual kernels (the face-flux kernel, the adjoint kernels and Euler stay).
-template <typename TC, int N>
-void useTensorKernels(Launchers& l) {
-  constexpr int EPB = sdg::TensorShape<N>::EPB, TPB = sdg::TensorShape<N>::TPB;
-  l.ns_grad_br1 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    hipLaunchKernelGGL((sdg::nsGradTensor<TC, N, 1>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a);
-  };
-  l.ns_grad_br2 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    hipLaunchKernelGGL((sdg::nsGradTensor<TC, N, 2>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a);
-  };
-  // face fluxes from the elements' own normal viscous fluxes (written by the gradient kernel)
-  l.ns_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    constexpr int NFQ = N * N;
-    hipLaunchKernelGGL((sdg::nsFaceFluxKernel<TC, 3, 6, NFQ, true>), dim3(blocksFor((g.F + g.Fb) * NFQ, sdg::kThreads)),
-                       dim3(sdg::kThreads), 0, st, g, ph, a);
-  };
-  l.ns_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    hipLaunchKernelGGL((sdg::nsResidualTensor<TC, N>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph,
-                       a);
-  };
-  l.trace = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const sdg::MixRef& mix) {
-    hipLaunchKernelGGL((sdg::tensorTraceKernel<TC, N>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, U,
-                       Uf, mix);
-  };
-  // the transpose of these stage kernels, FP64 in both precision modes: a mixed-precision context's
-  // adjoint differentiates the FP64 residual at the states of its run, on FP64 traces (trace64)
-  l.trace64 = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const sdg::MixRef& mix) {
-    hipLaunchKernelGGL((sdg::tensorTraceKernel<double, N>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, U, Uf, mix);
-  };
-  l.adj_volume[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-    hipLaunchKernelGGL((sdg::nsAdjVolumeTensor<N, 1>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a, j);
-  };
-  l.adj_volume[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-    hipLaunchKernelGGL((sdg::nsAdjVolumeTensor<N, 2>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a, j);
-  };
-  l.adj_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-    constexpr int NFQ = N * N;
-    if (ph.flux <= SDG_FLUX_ROE)
-      hipLaunchKernelGGL((sdg::nsAdjFaceRevKernel<3, 6, NFQ>), dim3(blocksFor(g.F * NFQ, sdg::kThreads)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a, j);
-    else
-      hipLaunchKernelGGL((sdg::nsAdjFaceKernel<3, 6, NFQ>), dim3(blocksFor(g.F * NFQ * 2 * 6, sdg::kThreads)),
-                         dim3(sdg::kThreads), 0, st, g, ph, a, j);
-  };
-  l.adj_lift[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-    hipLaunchKernelGGL((sdg::nsAdjLiftTensor<N, 1>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a, j);
-  };
-  l.adj_lift[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-    hipLaunchKernelGGL((sdg::nsAdjLiftTensor<N, 2>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a, j);
-  };
-  l.adj_gather = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const sdg::AdjArgs& j) {
-    hipLaunchKernelGGL((sdg::nsAdjGatherTensor<N>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a, j);
-  };
-  l.tensor = true;
-}
-// Navier-Stokes (BR1 or BR2, FP64 or mixed) with artificial viscosity on the sum-factorised kernels: the
-// gradient kernel adds eps grad U (the volume gradient) to the volume flux and to each side's normal
-// viscous flux, boundary points keep the volume-gradient trace (GfV) for the boundary flux
-template <typename TC, int N>
-void useTensorAvKernels(Launchers& l) {
-  constexpr int EPB = sdg::TensorShape<N>::EPB, TPB = sdg::TensorShape<N>::TPB;
-  l.av_ns_grad[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    hipLaunchKernelGGL((sdg::nsGradTensor<TC, N, 1, true>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a);
-  };
-  l.av_ns_grad[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    hipLaunchKernelGGL((sdg::nsGradTensor<TC, N, 2, true>), dim3(blocksFor(g.E, EPB)), dim3(TPB), 0, st, g, ph, a);
-  };
-  l.ns_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-    constexpr int NFQ = N * N;
-    hipLaunchKernelGGL((sdg::nsFaceFluxKernel<TC, 3, 6, NFQ, true, true>),
-                       dim3(blocksFor((g.F + g.Fb) * NFQ, sdg::kThreads)), dim3(sdg::kThreads), 0, st, g, ph, a);
-  };
-  l.av_ns_flux = l.ns_flux;
-}
-template <typename TC>
-bool selectTensorAvT(int order, Launchers& l) {
-  switch (order) {
-    case 2: useTensorAvKernels<TC, 3>(l); return true;
-    case 3: useTensorAvKernels<TC, 4>(l); return true;
-    case 4: useTensorAvKernels<TC, 5>(l); return true;
+bool selectLaunchers(int type, int order, bool force_valu, bool mixed, Launchers& l, bool tensor = false) {
+  switch (type) {
+    case SDG_ELEM_LINE: return sdg::selectLine(order, mixed, l);
+    case SDG_ELEM_TRIANGLE: return sdg::selectTriangle(order, mixed, l);
+    case SDG_ELEM_QUADRANGLE: return sdg::selectQuadrangle(order, force_valu, mixed, l);
+    case SDG_ELEM_TETRAHEDRON: return sdg::selectTetrahedron(order, force_valu, mixed, l);
+    case SDG_ELEM_PYRAMID: return sdg::selectPyramid(order, mixed, l);
+    case SDG_ELEM_HEXAHEDRON:
+      if (!sdg::selectHexahedron(order, force_valu, mixed, l)) return false;
+      return !tensor || force_valu || order < 2 || order > 4 || sdg::selectTensor(order, mixed, l);
     default: return false;
   }
 }
-bool selectTensorAv(int order, bool mixed, Launchers& l) {
-  return mixed ? selectTensorAvT<float>(order, l) : selectTensorAvT<double>(order, l);
-}
 
-template <int N>
-bool pickTensor(bool mixed, Launchers& l) {
-  if (mixed)
-    useTensorKernels<float, N>(l);
-  else
-    useTensorKernels<double, N>(l);
-  return true;
-}
-
-bool selectLaunchers(int type, int order, bool force_valu, bool mixed, Launchers& l, bool tensor = false) {
-  if (type == SDG_ELEM_HEXAHEDRON && tensor && !force_valu && order >= 2 && order <= 4) {
-    if (!selectLaunchers(type, order, false, mixed, l)) return false;
-    switch (order) {
-      case 2: return pickTensor<3>(mixed, l);
-      case 3: return pickTensor<4>(mixed, l);
-      default: return pickTensor<5>(mixed, l);
-    }
-  }
-  if (type == SDG_ELEM_LINE) {  // 1-D: vector kernels (P+1 modes, P+1 Gauss points, two end-point faces)
-    switch (order) {
-      case 1: return pickValu<1, 2, 2, 2, 1>(mixed, l);
-      case 2: return pickValu<1, 3, 3, 2, 1>(mixed, l);
-      case 3: return pickValu<1, 4, 4, 2, 1>(mixed, l);
-      case 4: return pickValu<1, 5, 5, 2, 1>(mixed, l);
-      case 5: return pickValu<1, 6, 6, 2, 1>(mixed, l);
-      default: return false;
-    }
-  }
-  if (type == SDG_ELEM_TRIANGLE) {  // bases of 3..15 functions: vector kernels
-    switch (order) {
-      case 1: return pickValu<2, 3, 3, 3, 2>(mixed, l);
-      case 2: return pickValu<2, 6, 6, 3, 3>(mixed, l);
-      case 3: return pickValu<2, 10, 12, 3, 4>(mixed, l);
-      case 4: return pickValu<2, 15, 16, 3, 5>(mixed, l);
-      default: return false;
-    }
-  }
-  if (type == SDG_ELEM_QUADRANGLE) {
-    switch (order) {
-      case 1: return pickValu<2, 4, 4, 4, 2>(mixed, l);
-      case 2: return pickValu<2, 9, 9, 4, 3>(mixed, l);
-      case 3: return pickMfma<2, 16, 16, 4, 4>(force_valu, mixed, l);
-      case 4: return pickMfma<2, 25, 25, 4, 5>(force_valu, mixed, l);
-      case 5: return pickMfma<2, 36, 36, 4, 6>(force_valu, mixed, l);
-      default: return false;
-    }
-  }
-  if (type == SDG_ELEM_TETRAHEDRON) {  // bases of 4..35 functions, Grundmann-Moeller volume rules
-    switch (order) {
-      case 1: return pickTet<4, 5, 4>(force_valu, mixed, l);
-      case 2: return pickTet<10, 15, 7>(force_valu, mixed, l);
-      case 3: return pickTet<20, 35, 13>(force_valu, mixed, l);
-      case 4: return pickTet<35, 70, 19>(force_valu, mixed, l);
-      default: return false;
-    }
-  }
-  if (type == SDG_ELEM_PYRAMID) {  // (P+1)^3 collapsed points, five faces of (P+1)^2 slots: vector kernels
-    switch (order) {
-      case 1: return pickValu<3, 5, 8, 5, 4>(mixed, l);
-      case 2: return pickValu<3, 14, 27, 5, 9>(mixed, l);
-      case 3: return pickValu<3, 30, 64, 5, 16>(mixed, l);
-      case 4: return pickValu<3, 55, 125, 5, 25>(mixed, l);
-      default: return false;
-    }
-  }
-  if (type == SDG_ELEM_HEXAHEDRON) {
-    switch (order) {
-      case 1: return pickValu<3, 8, 8, 6, 4>(mixed, l);
-      case 2: return pickMfma<3, 27, 27, 6, 9>(force_valu, mixed, l);
-      case 3: return pickMfma<3, 64, 64, 6, 16>(force_valu, mixed, l);
-      case 4: return pickMfma<3, 125, 125, 6, 25>(force_valu, mixed, l);
-      default: return false;
-    }
-  }
-  return false;
-}
-
-// 1-D tables and node/face maps of the sum-factorised hexahedron kernels (see dg_tensor.hpp).
+// 1-D tables and node/face maps of the sum-factorised kernels (hexahedra: dg_tensor.hpp,
+// quadrangles: dg_quad.hpp).
 bool buildTensorTables(const sdg::RefElement& r, sdg::TensorOps& t, std::vector<short>& perm, std::vector<short>& iperm,
                        std::vector<short>& slot_of, std::vector<short>& base, std::vector<double>& fwt) {
-  const int N = r.order + 1, NPT = N * N * N, NFQ = r.nfq;
-  if (r.type != SDG_ELEM_HEXAHEDRON || N > sdg::kTensorMaxN || r.nb != NPT || r.nq != NPT || NFQ != N * N) return false;
+  const int N = r.order + 1, D = r.type == SDG_ELEM_HEXAHEDRON ? 3 : 2, NF = 2 * D;
+  const int NFQ = D == 3 ? N * N : N, NPT = N * NFQ;
+  if ((r.type != SDG_ELEM_HEXAHEDRON && r.type != SDG_ELEM_QUADRANGLE) || N > sdg::kTensorMaxN || r.nb != NPT ||
+      r.nq != NPT || r.nfq != NFQ)
+    return false;
   std::vector<double> gx, gw;
   sdg::gaussLegendre(N, gx, gw);
   t = sdg::TensorOps{};
@@ -469,20 +100,20 @@ bool buildTensorTables(const sdg::RefElement& r, sdg::TensorOps& t, std::vector<
   perm.assign(NPT, 0);
   iperm.assign(NPT, 0);
   for (int b = 0; b < NPT; b++) {
-    const int tq = r.modes[b][0] + N * r.modes[b][1] + N * N * r.modes[b][2];
+    const int tq = r.modes[b][0] + N * r.modes[b][1] + (D == 3 ? N * N * r.modes[b][2] : 0);
     perm[b] = static_cast<short>(tq);
     iperm[tq] = static_cast<short>(b);
   }
-  slot_of.assign(static_cast<size_t>(6) * NPT, -1);
-  base.assign(static_cast<size_t>(6) * NFQ, -1);
-  fwt.assign(static_cast<size_t>(6) * NFQ, 0.0);
+  slot_of.assign(static_cast<size_t>(NF) * NPT, -1);
+  base.assign(static_cast<size_t>(NF) * NFQ, -1);
+  fwt.assign(static_cast<size_t>(NF) * NFQ, 0.0);
   const int stride[3] = {1, N, N * N};
-  for (int s = 0; s < 6; s++) {
-    const double* fp = &r.face_param[static_cast<size_t>(s) * NFQ * 3];
+  for (int s = 0; s < NF; s++) {
+    const double* fp = &r.face_param[static_cast<size_t>(s) * NFQ * D];
     int ax = -1;
-    for (int d = 0; d < 3 && ax < 0; d++) {
+    for (int d = 0; d < D && ax < 0; d++) {
       bool on = true;
-      for (int p = 0; p < NFQ; p++) on = on && std::fabs(std::fabs(fp[p * 3 + d]) - 1.0) < 1e-12 && fp[p * 3 + d] * fp[d] > 0.0;
+      for (int p = 0; p < NFQ; p++) on = on && std::fabs(std::fabs(fp[p * D + d]) - 1.0) < 1e-12 && fp[p * D + d] * fp[d] > 0.0;
       if (on) ax = d;
     }
     if (ax < 0) return false;
@@ -490,9 +121,9 @@ bool buildTensorTables(const sdg::RefElement& r, sdg::TensorOps& t, std::vector<
     t.side[s] = fp[ax] > 0.0 ? 1 : 0;
     for (int p = 0; p < NFQ; p++) {
       int bq = 0;
-      for (int d = 0; d < 3; d++) {
+      for (int d = 0; d < D; d++) {
         if (d == ax) continue;
-        const int i = nodeOf(fp[p * 3 + d]);
+        const int i = nodeOf(fp[p * D + d]);
         if (i < 0) return false;
         bq += i * stride[d];
       }
@@ -603,7 +234,7 @@ struct sdg_ctx {
   std::vector<double> h_lsq, h_V, h_chol;
   std::vector<int> h_bparent;  // parent element of each boundary face
   double* GfV = nullptr;  // Navier-Stokes with artificial viscosity: volume-gradient traces
-  double *U = nullptr, *Un = nullptr, *Uf[2] = {nullptr, nullptr}, *Gf = nullptr, *Rvol = nullptr, *Hs = nullptr, *Fv = nullptr,
+  double *U = nullptr, *Us = nullptr, *Uf[2] = {nullptr, nullptr}, *Gf = nullptr, *Rvol = nullptr, *Hs = nullptr, *Fv = nullptr,
          *Vn = nullptr, *Rsrc = nullptr, *src_li = nullptr;
   double *Rout = nullptr, *Wout = nullptr, *mon = nullptr, *rel = nullptr, *dtbuf = nullptr;
   int* status = nullptr;
@@ -736,7 +367,8 @@ void destroyGraphs(sdg_ctx* ctx) {
 StageArgs baseArgs(sdg_ctx* ctx) {
   StageArgs a{};
   a.U = ctx->U;
-  a.Un = ctx->Un;
+  a.Un = ctx->U;
+  a.Uo = ctx->U;
   a.Uf_in = ctx->Uf[ctx->cur];
   a.Uf_out = ctx->Uf[ctx->cur ^ 1];
   a.Gf = ctx->Gf;
@@ -771,6 +403,12 @@ void enqueueStage(sdg_ctx* ctx, int stage, double dt, int mode, double* wout, hi
   a.c2dt = c[2] * dt;
   a.last_stage = (stage == ctx->stages() - 1) ? 1 : 0;
   a.mode = mode;
+  // The step-start state stays in U until the last stage replaces it; the stages between work in Us.
+  // A second copy of the start state would cost a read in the first stage and a write in the last.
+  if (mode == 0) {
+    if (stage > 0) a.U = ctx->Us;
+    if (!a.last_stage) a.Uo = ctx->Us;
+  }
   if (ctx->recording && mode == 0) {
     a.rec = ctx->adj_pool;
     a.rec_t = ctx->mixed ? nullptr : ctx->adj_tpool;  // a mixed run's traces are FP32 deviations
@@ -782,7 +420,7 @@ void enqueueStage(sdg_ctx* ctx, int stage, double dt, int mode, double* wout, hi
   }
   a.Wout = wout;
   if (mode == 1) a.status = nullptr;
-  if (ctx->Rsrc) ctx->launch.source(ctx->stream, ctx->geo, ctx->phys, ctx->U, ctx->Rsrc, ctx->src_li);
+  if (ctx->Rsrc) ctx->launch.source(ctx->stream, ctx->geo, ctx->phys, a.U, ctx->Rsrc, ctx->src_li);
   if (ev) (void)hipEventRecord(ev[0], ctx->stream);
   if (ctx->ns()) {
     if (ctx->av)
@@ -1037,7 +675,12 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
                              "hexahedron P2-P4)"
                            : "sdg_create: no kernel instantiation for this element type and order");
   }
-  if (tensor_av && !selectTensorAv(r.order, mixed, ctx->launch)) {
+  if (r.type == SDG_ELEM_QUADRANGLE && problem->kernels == SDG_KERNELS_AUTO && !curved && !mixed && !av_vector &&
+      !sdg::selectQuadTensor(r.order, ctx->launch)) {
+    delete ctx;
+    return fail(nullptr, SDG_E_UNSUPPORTED, "sdg_create: no kernel instantiation for this element type and order");
+  }
+  if (tensor_av && !sdg::selectTensorAv(r.order, mixed, ctx->launch)) {
     delete ctx;
     return fail(nullptr, SDG_E_UNSUPPORTED, "sdg_create: no sum-factorised artificial-viscosity kernels for this order");
   }
@@ -1184,7 +827,8 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   }
   ctx->Fb = Fb;
   Geo& g = ctx->geo;
-  if (ctx->launch.tensor) {  // per slot normal and face weight for the sum-factorised kernels
+  const bool sum_fact = ctx->launch.tensor || ctx->launch.quad;  // sum-factorised stage kernels
+  if (sum_fact) {  // per slot normal and face weight
     std::vector<double> snrm(static_cast<size_t>(E) * naq * D), sjw(static_cast<size_t>(E) * naq);
     for (size_t o = 0; o < sjw.size(); o++) {
       if (snb[o] < 0) {
@@ -1399,11 +1043,11 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     g.op.lift = pl;
     g.op.rinterp = pi;
   }
-  if (ctx->launch.tensor) {
+  if (sum_fact) {
     std::vector<short> perm, iperm, slot_of, base;
     std::vector<double> fwt;
     if (!buildTensorTables(r, g.tens, perm, iperm, slot_of, base, fwt))
-      return bail(fail(ctx, SDG_E_INVALID, "sdg_create: inconsistent hexahedron tables for the sum-factorised kernels"));
+      return bail(fail(ctx, SDG_E_INVALID, "sdg_create: inconsistent element tables for the sum-factorised kernels"));
     short *dp, *dip, *ds, *db;
     double* dw;
     if (upload(ctx, perm, &dp) || upload(ctx, iperm, &dip) || upload(ctx, slot_of, &ds) || upload(ctx, base, &db) ||
@@ -1416,10 +1060,10 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     g.tens.fwt = dw;
     if (ctx->av) {  // P1 nodal functions at the tensor-ordered nodes (node artificial viscosity)
       const int N = r.order + 1;
-      std::vector<double> gx, gw, nodt(static_cast<size_t>(N) * N * N * r.nvert);
+      std::vector<double> gx, gw, nodt(static_cast<size_t>(nb) * r.nvert);
       sdg::gaussLegendre(N, gx, gw);
-      for (int q = 0; q < N * N * N; q++) {
-        const double xi[3] = {gx[q % N], gx[(q / N) % N], gx[q / (N * N)]};
+      for (int q = 0; q < nb; q++) {
+        const double xi[3] = {gx[q % N], gx[(q / N) % N], D == 3 ? gx[q / (N * N)] : 0.0};
         sdg::nodalValues(r, xi, &nodt[static_cast<size_t>(q) * r.nvert]);
       }
       double* dn;
@@ -1460,24 +1104,26 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   if (ctx->mixed ? (allocate(ctx, nUf, &ctx->Uf32[0]) || allocate(ctx, nUf, &ctx->Uf32[1]))
                  : (allocate(ctx, nUf, &ctx->Uf[0]) || allocate(ctx, nUf, &ctx->Uf[1])))
     return bail(SDG_E_NOMEM);
-  if (allocate(ctx, nU, &ctx->U) || allocate(ctx, nU, &ctx->Un) || allocate(ctx, nU, &ctx->Rout) ||
+  if (allocate(ctx, nU, &ctx->U) || allocate(ctx, nU, &ctx->Us) || allocate(ctx, nU, &ctx->Rout) ||
       allocate(ctx, (static_cast<size_t>(E) + sdg::kMonitorBlocks) * ctx->nv, &ctx->mon) || allocate(ctx, static_cast<size_t>(ctx->nv), &ctx->rel) ||
       allocate(ctx, static_cast<size_t>(E), &ctx->dtbuf) || allocate(ctx, size_t(2), &ctx->status))
     return bail(SDG_E_NOMEM);
   if (ctx->ns()) {
     const size_t nGf = static_cast<size_t>(E) * ctx->ng * naq, nFv = static_cast<size_t>(E) * nq * D * ctx->nv;
-    const bool tensor = ctx->launch.tensor;  // sum-factorised: Vn and the weak divergence Rvol, no Fv
+    const bool tensor = sum_fact;  // Vn and the weak divergence Rvol, no Fv
     if (ctx->mixed) {
       if (allocate(ctx, nGf, &ctx->Gf32) || allocate(ctx, nUf, &ctx->Hs32) || (!tensor && allocate(ctx, nFv, &ctx->Fv32)))
         return bail(SDG_E_NOMEM);
     } else {
-      if (allocate(ctx, nGf, &ctx->Gf) || allocate(ctx, nUf, &ctx->Hs)) return bail(SDG_E_NOMEM);
+      if (allocate(ctx, nGf, &ctx->Gf) || (!ctx->launch.quad && allocate(ctx, nUf, &ctx->Hs))) return bail(SDG_E_NOMEM);
       if (!tensor && (ctx->launch.mfma ? allocate(ctx, nFv, &ctx->Fv) : allocate(ctx, nU, &ctx->Rvol)))
         return bail(SDG_E_NOMEM);
     }
     if (tensor && (allocate(ctx, nUf, &ctx->Vn) || allocate(ctx, nU, &ctx->Rvol))) return bail(SDG_E_NOMEM);
   }
-  if (ctx->av && !ctx->ns() && !ctx->mixed &&
+  if (ctx->av && !ctx->ns() && ctx->launch.quad && (allocate(ctx, nUf, &ctx->Vn) || allocate(ctx, nU, &ctx->Rvol)))
+    return bail(SDG_E_NOMEM);
+  if (ctx->av && !ctx->ns() && !ctx->mixed && !ctx->launch.quad &&
       (allocate(ctx, static_cast<size_t>(E) * ctx->ng * naq, &ctx->Gf) ||
        (ctx->launch.mfma ? (allocate(ctx, nUf, &ctx->Hs) || allocate(ctx, static_cast<size_t>(E) * nq * D * ctx->nv, &ctx->Fv))
                          : allocate(ctx, nU, &ctx->Rvol))))
@@ -1490,7 +1136,7 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   if (ctx->av && ctx->ns() && allocate(ctx, static_cast<size_t>(E) * ctx->ng * naq, &ctx->GfV)) return bail(SDG_E_NOMEM);
   // modal Boussinesq source for the kernel sets that take it from a buffer (the sum-factorised
   // kernels form it at their nodes)
-  if (ctx->phys.source != SDG_SOURCE_NONE && !ctx->launch.tensor) {
+  if (ctx->phys.source != SDG_SOURCE_NONE && !sum_fact) {
     if (allocate(ctx, static_cast<size_t>(E) * ctx->nb, &ctx->Rsrc)) return bail(SDG_E_NOMEM);
     if (ctx->mixed && upload(ctx, r.mass_chol_inverse, &ctx->src_li)) return bail(SDG_E_NOMEM);
   }
@@ -1524,7 +1170,6 @@ int sdg_set_state(sdg_ctx* ctx, const double* coefficients) {
   HIP_TRY(ctx, hipMemcpyAsync(ctx->Rout, coefficients, bytes, hipMemcpyHostToDevice, ctx->stream));
   hipLaunchKernelGGL(referenceToDeviceKernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, ctx->stream,
                      ctx->Rout, ctx->U, ctx->E, ctx->nv, ctx->nb);
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->Un, ctx->U, bytes, hipMemcpyDeviceToDevice, ctx->stream));
   ctx->cur = 0;
   updateReference(ctx, coefficients);
   ctx->launch.trace(ctx->stream, ctx->geo, ctx->U, ctx->traces(0), ctx->mix);
@@ -1958,7 +1603,6 @@ int vjpAt(sdg_ctx* ctx, const double* U, double* lam, int apply_minv, double* ou
 int loadState(sdg_ctx* ctx, const double* src) {
   const size_t bytes = stateCount(ctx) * sizeof(double);
   HIP_TRY(ctx, hipMemcpyAsync(ctx->U, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->Un, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
   ctx->launch.trace(ctx->stream, ctx->geo, ctx->U, ctx->traces(ctx->cur), ctx->mix);
   HIP_TRY(ctx, hipGetLastError());
   return SDG_OK;
@@ -1987,8 +1631,8 @@ int saveState(sdg_ctx* ctx, double* dst) {
 // Stage s maps U_s to U_{s+1} = c0 U_0 + c1 U_s + c2 dt L(U_s) (TimeIntegration.cpp:45-65,181-198),
 // so its transpose is lam_s = c1 lam_{s+1} + c2 dt L'(U_s)^T lam_{s+1}, plus c0 lam_{s+1} to U_0.
 // The body of one adjoint step, starting from the state in adj_S[0]: recompute the stage states,
-// then transpose the stages in reverse order. The state buffers and trace parity it leaves behind
-// are those of S - 1 forward stages. No memset (the body is captured in a graph).
+// then transpose the stages in reverse order. The trace parity it leaves behind is that of S - 1
+// forward stages. No memset (the body is captured in a graph).
 int enqueueAdjointStep(sdg_ctx* ctx) {
   const int S = ctx->stages();
   int rc = loadState(ctx, ctx->adj_S[0]);
@@ -1996,7 +1640,8 @@ int enqueueAdjointStep(sdg_ctx* ctx) {
   hipLaunchKernelGGL(sdg::resetStatusKernel, dim3(1), dim3(64), 0, ctx->stream, ctx->status);
   for (int s = 0; s + 1 < S; s++) {
     enqueueStage(ctx, s, ctx->adj_dt, 0, nullptr);
-    if ((rc = saveState(ctx, ctx->adj_S[s + 1]))) return rc;
+    HIP_TRY(ctx, hipMemcpyAsync(ctx->adj_S[s + 1], ctx->Us, stateCount(ctx) * sizeof(double), hipMemcpyDeviceToDevice,
+                                ctx->stream));
   }
   for (int s = S - 1; s >= 0; s--)
     if ((rc = vjpAt(ctx, ctx->adj_S[s], ctx->adj_lam, 1, nullptr, s))) return rc;
