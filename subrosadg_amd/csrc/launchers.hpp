@@ -207,8 +207,8 @@ Launchers makeLaunchers() {
   l.monitor = [](hipStream_t st, const double* mon, int E, double* rel, int* status) {
     // mon holds E x NV per-element values followed by kMonitorBlocks x NV partial sums
     double* part = const_cast<double*>(mon) + static_cast<int64_t>(E) * (D + 2);
-    hipLaunchKernelGGL((monitorPartialKernel<D + 2>), dim3(kMonitorBlocks), dim3(kThreads), 0, st, mon, E, part, status);
-    hipLaunchKernelGGL((monitorKernel<D + 2>), dim3(1), dim3(kThreads), 0, st, part, E, rel, status);
+    hipLaunchKernelGGL((monitorKernel<D + 2>), dim3(monitorBlocks(E, D + 2)), dim3(kThreads), 0, st, mon, E, part, rel,
+                       status);
   };
   return l;
 }
@@ -222,11 +222,11 @@ bool pickMfma(bool force_valu, bool mixed, Launchers& l) {
     l = force_valu ? makeLaunchers<D, NB, NQ, NF, NFQ, false>() : makeLaunchers<D, NB, NQ, NF, NFQ, true>();
   return true;
 }
-// Tetrahedra: the FP64 matrix-core kernels, without the mixed mode and the adjoint of pickMfma
-template <int NB, int NQ, int NFQ>
-bool pickTet(bool force_valu, bool mixed, Launchers& l) {
+// Simplices: the FP64 matrix-core kernels, without the mixed mode and the adjoint of pickMfma
+template <int D, int NB, int NQ, int NF, int NFQ>
+bool pickSimplex(bool force_valu, bool mixed, Launchers& l) {
   if (mixed) return false;
-  l = force_valu ? makeLaunchers<3, NB, NQ, 4, NFQ, false>() : makeLaunchers<3, NB, NQ, 4, NFQ, true, double, false>();
+  l = force_valu ? makeLaunchers<D, NB, NQ, NF, NFQ, false>() : makeLaunchers<D, NB, NQ, NF, NFQ, true, double, false>();
   return true;
 }
 template <int D, int NB, int NQ, int NF, int NFQ>
@@ -363,7 +363,7 @@ bool pickTensor(bool mixed, Launchers& l) {
 
 // Kernel set of an element type and order; false where there is none. force_valu: the vector kernels.
 bool selectLine(int order, bool mixed, Launchers& l);
-bool selectTriangle(int order, bool mixed, Launchers& l);
+bool selectTriangle(int order, bool force_valu, bool mixed, Launchers& l);
 bool selectQuadrangle(int order, bool force_valu, bool mixed, Launchers& l);
 bool selectTetrahedron(int order, bool force_valu, bool mixed, Launchers& l);
 bool selectPyramid(int order, bool mixed, Launchers& l);

@@ -15,13 +15,13 @@ bool selectLine(int order, bool mixed, Launchers& l) {
   }
 }
 
-// bases of 3..15 functions: vector kernels
-bool selectTriangle(int order, bool mixed, Launchers& l) {
+// bases of 3..15 functions
+bool selectTriangle(int order, bool force_valu, bool mixed, Launchers& l) {
   switch (order) {
-    case 1: return pickValu<2, 3, 3, 3, 2>(mixed, l);
-    case 2: return pickValu<2, 6, 6, 3, 3>(mixed, l);
-    case 3: return pickValu<2, 10, 12, 3, 4>(mixed, l);
-    case 4: return pickValu<2, 15, 16, 3, 5>(mixed, l);
+    case 1: return pickSimplex<2, 3, 3, 3, 2>(force_valu, mixed, l);
+    case 2: return pickSimplex<2, 6, 6, 3, 3>(force_valu, mixed, l);
+    case 3: return pickSimplex<2, 10, 12, 3, 4>(force_valu, mixed, l);
+    case 4: return pickSimplex<2, 15, 16, 3, 5>(force_valu, mixed, l);
     default: return false;
   }
 }

@@ -31,7 +31,7 @@ namespace {
 bool selectLaunchers(int type, int order, bool force_valu, bool mixed, Launchers& l, bool tensor = false) {
   switch (type) {
     case SDG_ELEM_LINE: return sdg::selectLine(order, mixed, l);
-    case SDG_ELEM_TRIANGLE: return sdg::selectTriangle(order, mixed, l);
+    case SDG_ELEM_TRIANGLE: return sdg::selectTriangle(order, force_valu, mixed, l);
     case SDG_ELEM_QUADRANGLE: return sdg::selectQuadrangle(order, force_valu, mixed, l);
     case SDG_ELEM_TETRAHEDRON: return sdg::selectTetrahedron(order, force_valu, mixed, l);
     case SDG_ELEM_PYRAMID: return sdg::selectPyramid(order, mixed, l);
@@ -1106,7 +1106,7 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     return bail(SDG_E_NOMEM);
   if (allocate(ctx, nU, &ctx->U) || allocate(ctx, nU, &ctx->Us) || allocate(ctx, nU, &ctx->Rout) ||
       allocate(ctx, (static_cast<size_t>(E) + sdg::kMonitorBlocks) * ctx->nv, &ctx->mon) || allocate(ctx, static_cast<size_t>(ctx->nv), &ctx->rel) ||
-      allocate(ctx, static_cast<size_t>(E), &ctx->dtbuf) || allocate(ctx, size_t(2), &ctx->status))
+      allocate(ctx, static_cast<size_t>(E), &ctx->dtbuf) || allocate(ctx, size_t(4), &ctx->status))
     return bail(SDG_E_NOMEM);
   if (ctx->ns()) {
     const size_t nGf = static_cast<size_t>(E) * ctx->ng * naq, nFv = static_cast<size_t>(E) * nq * D * ctx->nv;
