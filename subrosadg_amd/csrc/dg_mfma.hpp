@@ -704,7 +704,7 @@ __global__ __launch_bounds__(kThreads) void nsFaceFluxKernel(Geo g, Phys ph, Sta
   double wl[D + 3], wr[D + 3], n[D], h[NV];
   computational<D>(ph, ul, wl);
   computational<D>(ph, ur, wr);
-  for (int d = 0; d < D; d++) n[d] = g.fnormal[(f * NFQ + j) * D + d];
+  for (int d = 0; d < D; d++) n[d] = g.fgeo[f * (D + 1) + d];  // straight faces
   convectiveFlux<D>(ph, n, ul, wl, ur, wr, h);
   if constexpr (sizeof(TC) == 4) reduceFaceFlux<D>(a, n, h);
   // normal viscous flux of each side, one side at a time (keeps one side's gradient live)
@@ -749,7 +749,7 @@ __global__ __launch_bounds__(kThreads) void nsFaceFluxKernel(Geo g, Phys ph, Sta
       }
     }
   }
-  const double jw = g.fjw[f * NFQ + j];
+  const double jw = g.fgeo[f * (D + 1) + D] * g.fwl[j];
   for (int v = 0; v < NV; v++) {
     const double t = (h[v] - (vl[v] + vr[v]) / 2.0) * jw;
     Hs[(L * NV + v) * NAQ + slL] = static_cast<TC>(-t);

@@ -159,8 +159,9 @@ __global__ __launch_bounds__(64) void quadGrad(Geo g, Phys ph, StageArgs a) {
   for (int v = 0; v < NV; v++) um[v] = a.U[(ec * NV + v) * NPT + q];
 #pragma unroll
   for (int v = 0; v < NV; v++) uo[v] = a.Uf_in[(ec * NV + v) * NAQ + sl];
-  for (int d = 0; d < D; d++) n[d] = g.snrm[es * D + d];
-  const double jw = g.sjw[es], dj = g.detj[ec];
+  const double* eg = g.egeo + (ec * 4 + sl / N) * 3;
+  for (int d = 0; d < D; d++) n[d] = eg[d];
+  const double jw = eg[2] * t.fwt[sl], dj = g.detj[ec];
   double gi[D * D];
   for (int i = 0; i < D * D; i++) gi[i] = g.ginv[ec * D * D + i];
   {
@@ -357,8 +358,9 @@ __global__ __launch_bounds__(64) void quadResidual(Geo g, Phys ph, StageArgs a) 
       rv[v] = a.Rvol[(ec * NV + v) * NPT + q];
     }
   }
-  for (int d = 0; d < D; d++) n[d] = g.snrm[es * D + d];
-  const double jw = g.sjw[es], dj = g.detj[ec];
+  const double* eg = g.egeo + (ec * 4 + sl / N) * 3;
+  for (int d = 0; d < D; d++) n[d] = eg[d];
+  const double jw = eg[2] * t.fwt[sl], dj = g.detj[ec];
   {
     const int64_t nb0 = nbs >= 0 ? static_cast<int64_t>(nbs / NAQ) * NV * NAQ + nbs % NAQ : ec * NV * NAQ + sl;
 #pragma unroll

@@ -179,19 +179,32 @@ __device__ __forceinline__ void loadModal(const TensorOps& t, const StageArgs& a
 template <typename TC, int N>
 __device__ __forceinline__ void writeTraces(const TensorLds<N>& L, const TC* sA, TC* Uf_out, int64_t e, int le, int tid,
                                             double* rec = nullptr) {
-  constexpr int NPT = N * N * N, NV = 5, NFQ = N * N, NAQ = 6 * NFQ, EPB = TensorShape<N>::EPB;
-  for (int idx = tid - le * NPT; idx < NAQ * NV; idx += NPT) {
-    if (idx < 0) break;
-    const int sl = idx % NAQ, v = idx / NAQ, s = sl / NFQ;
-    const int b = L.base[sl], st = axisStride(L.axis[s], N);
-    const TC* l = tabLf<TC, N>(L) + L.side[s] * N;
-    TC acc = TC(0);
+  constexpr int NPT = N * N * N, NV = 5, NFQ = N * N, NAQ = 6 * NFQ;
 #pragma unroll
-    for (int i = 0; i < N; i++) acc += l[i] * sA[v * NPT + b + i * st];
-    Uf_out[(e * NV + v) * NAQ + sl] = acc;
-    if (rec) rec[(e * NV + v) * NAQ + sl] = static_cast<double>(acc);
+  for (int k = 0; k < (NAQ + NPT - 1) / NPT; k++) {
+    const int sl = tid - le * NPT + k * NPT;
+    if (sl >= NAQ) break;
+    const int b = L.base[sl], s = sl / NFQ, st = axisStride(L.axis[s], N);
+    TC l[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) l[i] = tabLf<TC, N>(L)[L.side[s] * N + i];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      TC acc = TC(0);
+#pragma unroll
+      for (int i = 0; i < N; i++) acc += l[i] * sA[v * NPT + b + i * st];
+      Uf_out[(e * NV + v) * NAQ + sl] = acc;
+      if (rec) rec[(e * NV + v) * NAQ + sl] = static_cast<double>(acc);
+    }
   }
-  (void)EPB;
+}
+
+// the element's outward face normals and area factors, [face][normal, |J_f|], into LDS (the caller's
+// next workgroup barrier publishes them)
+template <int N>
+__device__ __forceinline__ void loadFaceGeometry(const Geo& g, int64_t e, double* sN, int q, bool ok) {
+  static_assert(N * N * N >= 24, "one value per lane");
+  if (ok && q < 24) sN[q] = g.egeo[e * 24 + q];
 }
 
 // element slot of a thread (tid / NPT); at NPT = 64 a wavefront is one element, and the index is
@@ -278,6 +291,10 @@ __device__ __forceinline__ void normalViscous32(const Phys& ph, const double* u,
 // faces' average traces, SpatialDiscrete.cpp:844-911: BR2's face-gradient field, the alpha lifts
 // alone under BR1) added to the volume flux and to each side's normal viscous flux
 // (ViscousFlux.cpp:105-190); boundary points keep its trace in GfV for the boundary flux
+// Latency bound: three workgroups fit a CU (LDS in FP64, registers), and half of the VALU and LDS issue
+// slots are used. Normals and face weights come from 24 doubles per element in LDS instead of a normal
+// and a weight per face point in HBM (a load and a wait per face): 32^3 P3 221 -> 190 us in FP64 and
+// 152 -> 125 us mixed, with the slots' own traces kept in registers.
 template <typename TC, int N, int VISC, bool AV = false>
 __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys ph, StageArgs a) {
   static_assert(!AV || VISC == 1 || VISC == 2, "artificial viscosity: BR1 / BR2");
@@ -287,6 +304,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
   static_assert(NV * NPT + NV * NAQ <= NG * NPT && NV * NPT <= NV * NAQ, "LDS regions do not nest");
   __shared__ TC sW[EPB][NG * NPT];
   __shared__ TC sB[EPB][NV * NAQ];
+  __shared__ double sN[EPB][24];
   __shared__ TensorLds<N> sT;
   if (a.status && a.status[0]) return;
   stageTables<N>(t, sT);
@@ -305,33 +323,30 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
     for (int i = 0; i < D * D; i++) gi[i] = g.ginv[e * D * D + i];
   }
   // face terms per (variable, slot): alpha = A - u_own n |J_f| w and beta = J (scalars of n_out).
-  // The interior faces' operands are gathered first, so that their latency overlaps the basis
-  // passes; boundary slots get jw = 0 here and are filled in after the passes.
+  // A lane takes the slots q, q + NPT of all variables: the neighbour index is read once per slot and
+  // the own traces stay in registers for the normal flux. All loads are issued here, branch-free, so
+  // that their latency overlaps the basis passes (a slot past the end reads slot 0, one on a
+  // boundary its own trace).
   const TC* Uf_in = pick<TC>(a.Uf_in, a.Uf_in32);
-  constexpr int ITEMS = (NV * NAQ + NPT - 1) / NPT;
-  TC fo[ITEMS], fn[ITEMS];
-  double fw[ITEMS];
+  constexpr int SI = (NAQ + NPT - 1) / NPT;
+  // at N = 5 in FP64 keeping them costs the third wavefront per SIMD (64 -> 71 us at 16^3): read again
+  constexpr bool KEEP = sizeof(TC) == 4 || N < 5;
+  TC fo[SI][NV], fn[SI][NV];
+  int nbk[SI];
+  loadFaceGeometry<N>(g, e, sN[lec], q, ok);
   if (ok) {
-    // branch-free: the neighbour slots first, then every trace and weight load at once (a slot
-    // past the end or on a boundary reads its own trace and gets weight 0)
-    int nbk[ITEMS];
 #pragma unroll
-    for (int k = 0; k < ITEMS; k++) {
-      const int idx = q + k * NPT;
-      nbk[k] = g.snb[e * NAQ + (idx < NV * NAQ ? idx % NAQ : 0)];
-    }
+    for (int k = 0; k < SI; k++) nbk[k] = g.snb[e * NAQ + (q + k * NPT < NAQ ? q + k * NPT : 0)];
 #pragma unroll
-    for (int k = 0; k < ITEMS; k++) {
-      const int idx = q + k * NPT;
-      const bool in = idx < NV * NAQ;
-      const int v = in ? idx / NAQ : 0, sl = in ? idx % NAQ : 0, nbs = nbk[k];
-      const bool inner = in && nbs >= 0;
-      const int64_t own = (e * NV + v) * NAQ + sl;
-      const int64_t nbr = inner ? (static_cast<int64_t>(nbs / NAQ) * NV + v) * NAQ + nbs % NAQ : own;
-      fo[k] = Uf_in[own];
-      fn[k] = Uf_in[nbr];
-      const double jw = g.sjw[e * NAQ + sl];
-      fw[k] = inner ? jw : 0.0;
+    for (int k = 0; k < SI; k++) {
+      const int sl = q + k * NPT < NAQ ? q + k * NPT : 0, nbs = nbk[k];
+      const int64_t own = e * NV * NAQ + sl;
+      const int64_t nbr = nbs >= 0 ? static_cast<int64_t>(nbs / NAQ) * NV * NAQ + nbs % NAQ : own;
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        fo[k][v] = Uf_in[own + v * NAQ];
+        fn[k][v] = Uf_in[nbr + v * NAQ];
+      }
     }
   }
   loadModal<TC, N>(t, a, a.U, e, Bt, q, ok);
@@ -342,36 +357,37 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
   elemSync<NPT>();
   linePass<TC, N, NV>(tabB<TC, N>(sT), 2, Bt, Y, q, ok);  // Y: nodal state
   elemSync<NPT>();
+  // an interior face's alpha = ((u_o + u_n)/2 - u_o) |J_f| w is its beta, so alpha is kept apart only
+  // on meshes with boundary faces
+  const bool bounded = g.Fb > 0;
   if (ok) {
 #pragma unroll
-    for (int k = 0; k < ITEMS; k++) {
-      const int idx = q + k * NPT;
-      if (idx < NV * NAQ) {
-        // in the contraction type (the FP64 mode's arithmetic is FP64; the mixed mode's traces
-        // are FP32 deviations already)
-        const TC uo = fo[k], un = fn[k], w = static_cast<TC>(fw[k]);
-        Al[idx] = ((uo + un) / TC(2) - uo) * w;
-        Bt[idx] = ((un - uo) / TC(2)) * w;
+    for (int k = 0; k < SI; k++) {
+      const int sl = q + k * NPT;
+      if (sl >= NAQ) break;
+      const int s = sl / NFQ;
+      if (nbk[k] >= 0) {
+        const TC w = static_cast<TC>(sN[lec][s * 4 + 3] * sT.fwt[sl]);
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+          const TC be = ((fn[k][v] - fo[k][v]) / TC(2)) * w;
+          Bt[v * NAQ + sl] = be;
+          if (bounded) Al[v * NAQ + sl] = be;
+        }
+      } else {  // boundary face point: the boundary condition's gradient states
+        const int bp = -1 - nbk[k];
+        const double jw = g.bjw[bp];
+        double ub[NV], wd[D + 3], n[D], uvg[NV], uig[NV];
+        for (int v = 0; v < NV; v++) ub[v] = pointState<TC>(a, fo[k][v], v);
+        for (int d = 0; d < D; d++) n[d] = g.bnormal[static_cast<int64_t>(bp) * D + d];
+        for (int i = 0; i < D + 3; i++) wd[i] = g.bdata[static_cast<int64_t>(bp) * (D + 3) + i];
+        boundaryGradientStates<D>(ph, g.btype[bp], n, ub, wd, uvg, uig);
+        for (int v = 0; v < NV; v++) {
+          Al[v * NAQ + sl] = static_cast<TC>((uvg[v] - ub[v]) * jw);
+          Bt[v * NAQ + sl] = static_cast<TC>(uig[v] * jw);
+        }
       }
     }
-    if (g.Fb > 0)
-      for (int idx = q; idx < NV * NAQ; idx += NPT) {
-        const int v = idx / NAQ, sl = idx % NAQ;
-        const int nbs = g.snb[e * NAQ + sl];
-        if (nbs >= 0) continue;
-        const double uo = Uf_in[(e * NV + v) * NAQ + sl];
-        double ub[NV], Ab[D], Jb[D];
-        for (int k = 0; k < NV; k++) ub[k] = pointState<TC>(a, Uf_in[(e * NV + k) * NAQ + sl], k);
-        boundaryGradientTerms<D>(ph, g, -1 - nbs, ub, v, sizeof(TC) == 4 ? a.mix.uref[v] : 0.0, Ab, Jb);
-        // A and J are (scalar) n |J_f| w; recover the scalars along the dominant normal component
-        const int bp = -1 - nbs;
-        int dm = 0;
-        for (int d = 1; d < D; d++)
-          if (fabs(g.bnormal[static_cast<int64_t>(bp) * D + d]) > fabs(g.bnormal[static_cast<int64_t>(bp) * D + dm])) dm = d;
-        const double nd = g.bnormal[static_cast<int64_t>(bp) * D + dm];
-        Al[idx] = static_cast<TC>(Ab[dm] / nd - uo * g.bjw[bp]);
-        Bt[idx] = static_cast<TC>(Jb[dm] / nd);
-      }
   }
   elemSync<NPT>();
   // gradient at the node: J^-T (Dn u along each axis) + the face corrections, assembled in the
@@ -400,28 +416,19 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
         if constexpr (VISC == 2 || AV) wface[v * D + d] = s;
       }
     }
-    // the outward normal at the node's face point, loaded one face ahead of its use
-    double nx[D];
-    {
-      const int64_t es = e * NAQ + sT.slot_of[q];
-      for (int d = 0; d < D; d++) nx[d] = g.snrm[es * D + d];
-    }
     const double inw = 1.0 / (sT.wn[q] * dj);  // M^-1 at the node, one reciprocal for the six faces
 #pragma unroll 1  // unrolled, the six faces' LDS loads are hoisted together and double the VGPRs
     for (int s = 0; s < 6; s++) {
       const int ax = t.axis[s], i = nodeIndex(q, ax, N);
       const int sl = s * NFQ + sT.slot_of[s * NPT + q];
       TC n[D];
-      for (int d = 0; d < D; d++) n[d] = static_cast<TC>(nx[d]);
-      if (s < 5) {
-        const int64_t es = e * NAQ + (s + 1) * NFQ + sT.slot_of[(s + 1) * NPT + q];
-        for (int d = 0; d < D; d++) nx[d] = g.snrm[es * D + d];
-      }
+      for (int d = 0; d < D; d++) n[d] = static_cast<TC>(sN[lec][s * 4 + d]);
       // alpha, beta carry |J_f| w_t1 w_t2; M^-1 = 1 / (w_i w_t1 w_t2 |J|) at the node
       const TC coef = static_cast<TC>(sT.lf[t.side[s] * N + i] * inw);
       for (int v = 0; v < NV; v++) {
-        const TC al = Al[v * NAQ + sl] * coef;
         const TC be = Bt[v * NAQ + sl] * coef;
+        TC al = be;
+        if (bounded) al = Al[v * NAQ + sl] * coef;
         for (int d = 0; d < D; d++) {
           wtot[v * D + d] += (al + be) * n[d];
           if constexpr (VISC == 2 || AV) wface[v * D + d] += al * n[d];
@@ -456,23 +463,21 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
   // BR1 with artificial viscosity: the AV term of each own slot's normal flux takes the volume
   // gradient's trace, which is not the field BR1's viscous flux traces, so it goes first: eps times
   // the trace . n per slot (NV values kept in registers) and, at boundary slots, the trace itself
-  constexpr int SI0 = (NAQ + NPT - 1) / NPT;
-  double avn[AV && VISC == 1 ? SI0 : 1][NV];
+  double avn[AV && VISC == 1 ? SI : 1][NV];
   if constexpr (AV && VISC == 1) {
     if (ok)
       for (int r = 0; r < NG; r++) W[r * NPT + q] = wface[r];
     elemSync<NPT>();
     if (ok) {
 #pragma unroll
-      for (int k = 0; k < SI0; k++) {
+      for (int k = 0; k < SI; k++) {
         const int sl = q + k * NPT;
         if (sl >= NAQ) break;
         const int s = sl / NFQ;
         const int b = sT.base[sl], st = axisStride(sT.axis[s], N);
-        const int64_t es = e * NAQ + sl;
-        const int nbs = g.snb[es];
+        const int nbs = nbk[k];
         double n[D];
-        for (int d = 0; d < D; d++) n[d] = g.snrm[es * D + d];
+        for (int d = 0; d < D; d++) n[d] = sN[lec][s * 4 + d];
         const TC* lt = tabLf<TC, N>(sT) + sT.side[s] * N;
         const double eps = avAt(g, g.nodf, sl, static_cast<int>(e));
         for (int v = 0; v < NV; v++) avn[k][v] = 0.0;
@@ -498,21 +503,11 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
   if (ok) {
     TC* Gf = pick<TC>(a.Gf, a.Gf32);
     const double idj = 1.0 / dj;
-    constexpr int SI = (NAQ + NPT - 1) / NPT;
-    // the slots' neighbour flags, normals and own traces, all gathered before the loop (a slot
-    // past the end reads slot 0)
-    int nbk[SI];
-    double nk[SI][D];
-    TC uk[SI][NV];
+    if constexpr (!KEEP) {
 #pragma unroll
-    for (int k = 0; k < SI; k++) {
-      const int sl = q + k * NPT < NAQ ? q + k * NPT : 0;
-      const int64_t es = e * NAQ + sl;
-      nbk[k] = g.snb[es];
+      for (int k = 0; k < SI; k++)
 #pragma unroll
-      for (int d = 0; d < D; d++) nk[k][d] = g.snrm[es * D + d];
-#pragma unroll
-      for (int v = 0; v < NV; v++) uk[k][v] = Uf_in[(e * NV + v) * NAQ + sl];
+        for (int v = 0; v < NV; v++) fo[k][v] = Uf_in[(e * NV + v) * NAQ + (q + k * NPT < NAQ ? q + k * NPT : 0)];
     }
 #pragma unroll
     for (int k = 0; k < SI; k++) {
@@ -522,8 +517,8 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsGradTensor(Geo g, Phys 
       const int b = sT.base[sl], st = axisStride(sT.axis[s], N);
       const int nbs = nbk[k];
       double n[D], us[NV], gs[NG];
-      for (int d = 0; d < D; d++) n[d] = nk[k][d];
-      for (int v = 0; v < NV; v++) us[v] = pointState<TC>(a, uk[k][v], v);
+      for (int d = 0; d < D; d++) n[d] = sN[lec][s * 4 + d];
+      for (int v = 0; v < NV; v++) us[v] = pointState<TC>(a, fo[k][v], v);
       // BR2 own-face lift factor of the slot, times the normal (in the contraction type)
       const double kf = sT.kappa[sT.side[s]] * idj / sT.fwt[sl];
       TC kn[D];
@@ -664,7 +659,6 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsResidualTensor(Geo g, P
                                                                               : NV * NPT * 8) / 8;
   __shared__ double sF[EPB][NV * NPT];  // FP64 scratch of the basis passes
   __shared__ double sHR[EPB][HB];
-  __shared__ double sM[EPB][NV];        // monitor partials
   __shared__ TensorLds<N> sT;
   if (a.status && a.status[0]) return;
   stageTables<N>(t, sT);
@@ -751,13 +745,20 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsResidualTensor(Geo g, P
     elemSync<NPT>();
     pass64(sT.B, false, 2, T0, SR);  // SR: R V^T at the nodes
     elemSync<NPT>();
-    if (le < EPB && q < NV) {
+    constexpr int GR = NPT / NV;  // lanes per variable, then one lane per variable
+    if (le < EPB && q < GR * NV) {
+      const int v = q / GR;
       double s = 0.0;
-      for (int k = 0; k < NPT; k++) s += fabs(SR[q * NPT + k]);
-      sM[le][q] = s;
+      for (int k = q % GR; k < NPT; k += GR) s += fabs(SR[v * NPT + k]);
+      T0[q] = s;
     }
     elemSync<NPT>();
-    if (ok && q < NV) a.mon[e * NV + q] = sM[le][q] / NPT;
+    if (ok && q < NV) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < GR; k++) s += T0[q * GR + k];
+      a.mon[e * NV + q] = s / NPT;
+    }
     // the nodal increment R_psi / (w |J|) from the registers (SR was overwritten)
     elemSync<NPT>();
     if (ok) {

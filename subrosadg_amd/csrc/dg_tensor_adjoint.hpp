@@ -69,6 +69,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB, 2) void nsAdjVolumeTensor(Geo 
   __shared__ double sW[EPB][NG * NPT];
   __shared__ double sB[EPB][NV * NAQ];
   __shared__ double sM[EPB][NV * NPT];
+  __shared__ double sN[EPB][24];
   __shared__ TensorLds<N> sT;
   stageTables<N>(t, sT);
   const int tid = threadIdx.x, le = localElement<NPT>(tid), q = tid % NPT;
@@ -82,21 +83,23 @@ __global__ __launch_bounds__(TensorShape<N>::TPB, 2) void nsAdjVolumeTensor(Geo 
   double* Mu = sM[lec];
   double dj = 1.0;
   if (ok) dj = g.detj[e];
-  constexpr int ITEMS = (NV * NAQ + NPT - 1) / NPT;
-  double fo[ITEMS], fn[ITEMS], fw[ITEMS];
+  // the forward kernel's loads (periodic meshes: every slot has a neighbour)
+  constexpr int SI = (NAQ + NPT - 1) / NPT;
+  double fo[SI][NV], fn[SI][NV];
+  loadFaceGeometry<N>(g, e, sN[lec], q, ok);
   if (ok) {
+    int nbk[SI];
 #pragma unroll
-    for (int k = 0; k < ITEMS; k++) {
-      const int idx = q + k * NPT;
-      const bool in = idx < NV * NAQ;
-      const int v = in ? idx / NAQ : 0, sl = in ? idx % NAQ : 0;
-      const int nbs = g.snb[e * NAQ + sl];
-      const bool inner = in && nbs >= 0;
-      const int64_t own = (e * NV + v) * NAQ + sl;
-      const int64_t nbr = inner ? (static_cast<int64_t>(nbs / NAQ) * NV + v) * NAQ + nbs % NAQ : own;
-      fo[k] = a.Uf_in[own];
-      fn[k] = a.Uf_in[nbr];
-      fw[k] = inner ? g.sjw[e * NAQ + sl] : 0.0;
+    for (int k = 0; k < SI; k++) nbk[k] = g.snb[e * NAQ + (q + k * NPT < NAQ ? q + k * NPT : 0)];
+#pragma unroll
+    for (int k = 0; k < SI; k++) {
+      const int64_t own = e * NV * NAQ + (q + k * NPT < NAQ ? q + k * NPT : 0);
+      const int64_t nbr = nbk[k] >= 0 ? static_cast<int64_t>(nbk[k] / NAQ) * NV * NAQ + nbk[k] % NAQ : own;
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        fo[k][v] = a.Uf_in[own + v * NAQ];
+        fn[k][v] = a.Uf_in[nbr + v * NAQ];
+      }
     }
   }
   loadModal<double, N>(t, a, a.U, e, Bt, q, ok);
@@ -132,12 +135,12 @@ __global__ __launch_bounds__(TensorShape<N>::TPB, 2) void nsAdjVolumeTensor(Geo 
   elemSync<NPT>();
   if (ok) {
 #pragma unroll
-    for (int k = 0; k < ITEMS; k++) {
-      const int idx = q + k * NPT;
-      if (idx < NV * NAQ) {
-        Al[idx] = ((fo[k] + fn[k]) / 2.0 - fo[k]) * fw[k];
-        Bt[idx] = ((fn[k] - fo[k]) / 2.0) * fw[k];
-      }
+    for (int k = 0; k < SI; k++) {
+      const int sl = q + k * NPT;
+      if (sl >= NAQ) break;
+      const double w = sN[lec][sl / NFQ * 4 + 3] * sT.fwt[sl];
+#pragma unroll
+      for (int v = 0; v < NV; v++) Bt[v * NAQ + sl] = ((fn[k][v] - fo[k][v]) / 2.0) * w;  // beta, and alpha: the same
     }
   }
   elemSync<NPT>();
@@ -174,10 +177,10 @@ __global__ __launch_bounds__(TensorShape<N>::TPB, 2) void nsAdjVolumeTensor(Geo 
       const int ax = t.axis[s], i = nodeIndex(q, ax, N);
       const int sl = s * NFQ + sT.slot_of[s * NPT + q];
       double n[D];
-      for (int d = 0; d < D; d++) n[d] = g.snrm[(e * NAQ + sl) * D + d];
+      for (int d = 0; d < D; d++) n[d] = sN[lec][s * 4 + d];
       const double coef = sT.lf[t.side[s] * N + i] * inw;
       for (int v = 0; v < NV; v++) {
-        const double al = Al[v * NAQ + sl] * coef, be = Bt[v * NAQ + sl] * coef;
+        const double be = Bt[v * NAQ + sl] * coef, al = be;
         for (int d = 0; d < D; d++) {
           gtot[v * D + d] += (al + be) * n[d];
           gface[v * D + d] += (VISC == 2 ? al : al + be) * n[d];
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB, 2) void nsAdjVolumeTensor(Geo 
       const double* l = sT.lf + sT.side[s] * N;
       const double kf = sT.kappa[sT.side[s]] * idj / sT.fwt[sl];
       double n[D];
-      for (int d = 0; d < D; d++) n[d] = g.snrm[(e * NAQ + sl) * D + d];
+      for (int d = 0; d < D; d++) n[d] = sN[lec][s * 4 + d];
       for (int r = 0; r < NG; r++) {
         double acc = 0.0;
 #pragma unroll
@@ -251,6 +254,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsAdjLiftTensor(Geo g, Ph
   using S = TensorShape<N>;
   constexpr int NPT = S::NPT, EPB = S::EPB, NV = S::NV, NG = S::NG, NFQ = S::NFQ, NAQ = S::NAQ, D = 3;
   __shared__ double sZ[EPB][NG * NPT];
+  __shared__ double sN[EPB][24];
   __shared__ TensorLds<N> sT;
   stageTables<N>(t, sT);
   const int tid = threadIdx.x, le = localElement<NPT>(tid), q = tid % NPT;
@@ -262,6 +266,7 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsAdjLiftTensor(Geo g, Ph
   for (int i = 0; i < D * D; i++) gi[i] = 0.0;
   double gt[NG], gf[NG];
   for (int r = 0; r < NG; r++) gt[r] = gf[r] = 0.0;
+  loadFaceGeometry<N>(g, e, sN[lec], q, ok);
   if (ok) {
     dj = g.detj[e];
     for (int i = 0; i < D * D; i++) gi[i] = g.ginv[e * D * D + i];
@@ -324,14 +329,14 @@ __global__ __launch_bounds__(TensorShape<N>::TPB) void nsAdjLiftTensor(Geo g, Ph
         double acc = 0.0;
 #pragma unroll
         for (int i = 0; i < N; i++) acc += l[i] * Z[(v * D + d) * NPT + b + i * st];
-        ab += acc * g.snrm[es * D + d];
+        ab += acc * sN[lec][s * 4 + d];
       }
       if constexpr (VISC == 2) {  // own-face lift: gs += kappa beta n / (|J| fw)
         const double kf = sT.kappa[sT.side[s]] * idj / sT.fwt[sl];
-        for (int d = 0; d < D; d++) ab += kf * j.GFb[(e * NG + v * D + d) * NAQ + sl] * g.snrm[es * D + d];
+        for (int d = 0; d < D; d++) ab += kf * j.GFb[(e * NG + v * D + d) * NAQ + sl] * sN[lec][s * 4 + d];
       }
       // alpha = beta = (u_n - u_o)/2 fw in their derivatives
-      const double sb = ab * (g.snb[es] >= 0 ? g.sjw[es] : 0.0) / 2.0;
+      const double sb = ab * (g.snb[es] >= 0 ? sN[lec][s * 4 + 3] * sT.fwt[sl] : 0.0) / 2.0;
       j.Pown[(e * NV + v) * NAQ + sl] = -sb;
       j.Qnb[(e * NV + v) * NAQ + sl] = sb;
     }

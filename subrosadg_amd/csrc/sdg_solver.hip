@@ -828,24 +828,36 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   ctx->Fb = Fb;
   Geo& g = ctx->geo;
   const bool sum_fact = ctx->launch.tensor || ctx->launch.quad;  // sum-factorised stage kernels
-  if (sum_fact) {  // per slot normal and face weight
-    std::vector<double> snrm(static_cast<size_t>(E) * naq * D), sjw(static_cast<size_t>(E) * naq);
-    for (size_t o = 0; o < sjw.size(); o++) {
-      if (snb[o] < 0) {
-        const size_t bp = static_cast<size_t>(-1 - snb[o]);
-        for (int d = 0; d < D; d++) snrm[o * D + d] = bnormal[bp * D + d];
-        sjw[o] = bjw[bp];
-      } else {
-        const size_t fp = static_cast<size_t>(sfp[o] >> 1);
-        const double sg = (sfp[o] & 1) ? -1.0 : 1.0;
-        for (int d = 0; d < D; d++) snrm[o * D + d] = sg * fnormal[fp * D + d];
-        sjw[o] = fjw[fp];
-      }
+  if (!curved) {  // straight faces: normal and area factor once per face, and per element face
+    std::vector<double> fgeo(static_cast<size_t>(ctx->F) * (D + 1));
+    for (int64_t f = 0; f < ctx->F; f++) {
+      for (int d = 0; d < D; d++) fgeo[f * (D + 1) + d] = fnormal[f * nfq * D + d];
+      fgeo[f * (D + 1) + D] = fjw[f * nfq] / r.fweight[0];
     }
-    double *dsn, *dsj;
-    if (upload(ctx, snrm, &dsn) || upload(ctx, sjw, &dsj)) return bail(SDG_E_NOMEM);
-    g.snrm = dsn;
-    g.sjw = dsj;
+    double *df, *dw;
+    if (upload(ctx, fgeo, &df) || upload(ctx, r.fweight, &dw)) return bail(SDG_E_NOMEM);
+    g.fgeo = df;
+    g.fwl = dw;
+    if (sum_fact) {
+      std::vector<double> egeo(static_cast<size_t>(E) * r.nf * (D + 1));
+      for (size_t o = 0; o < static_cast<size_t>(E) * r.nf; o++) {
+        double* eg = &egeo[o * (D + 1)];
+        const size_t sl = o * nfq;
+        if (snb[sl] < 0) {
+          const size_t bp = static_cast<size_t>(-1 - snb[sl]);
+          for (int d = 0; d < D; d++) eg[d] = bnormal[bp * D + d];
+          eg[D] = bjw[bp] / r.fweight[bp % nfq];
+        } else {
+          const size_t f = static_cast<size_t>(sfp[sl] >> 1) / nfq;
+          const double sg = (sfp[sl] & 1) ? -1.0 : 1.0;
+          for (int d = 0; d < D; d++) eg[d] = sg * fgeo[f * (D + 1) + d];
+          eg[D] = fgeo[f * (D + 1) + D];
+        }
+      }
+      double* de;
+      if (upload(ctx, egeo, &de)) return bail(SDG_E_NOMEM);
+      g.egeo = de;
+    }
   }
   double *dVt, *ddV, *dVft, *dVf, *dMinv, *dLf, *dwq, *dginv, *ddetj, *dnormal, *djw, *dme;
   int *dseq, *dseqinv, *dfpar, *dfloc, *dsnb, *dsfp, *dbtype, *dbslot;
@@ -935,7 +947,9 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     g.ntag = dtag;
     g.nodeav = ctx->nodeav;
   }
-  {
+  // padded operators of the matrix-core kernels (the sum-factorised quadrangles use them in the adjoint,
+  // on periodic Navier-Stokes meshes)
+  if (ctx->launch.mfma && (!ctx->launch.quad || (ctx->ns() && Fb == 0))) {
     const int nfq_ = nfq;
     auto V = [&](int q, int b) { return r.V[static_cast<size_t>(q) * nb + b]; };
     auto Vfv = [&](int sl, int b) { return r.Vf[static_cast<size_t>(sl) * nb + b]; };
@@ -1048,15 +1062,15 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     std::vector<double> fwt;
     if (!buildTensorTables(r, g.tens, perm, iperm, slot_of, base, fwt))
       return bail(fail(ctx, SDG_E_INVALID, "sdg_create: inconsistent element tables for the sum-factorised kernels"));
-    short *dp, *dip, *ds, *db;
+    std::vector<short> maps(perm);
+    for (const std::vector<short>* m : {&iperm, &slot_of, &base}) maps.insert(maps.end(), m->begin(), m->end());
+    short* dp;
     double* dw;
-    if (upload(ctx, perm, &dp) || upload(ctx, iperm, &dip) || upload(ctx, slot_of, &ds) || upload(ctx, base, &db) ||
-        upload(ctx, fwt, &dw))
-      return bail(SDG_E_NOMEM);
+    if (upload(ctx, maps, &dp) || upload(ctx, fwt, &dw)) return bail(SDG_E_NOMEM);
     g.tens.perm = dp;
-    g.tens.iperm = dip;
-    g.tens.slot_of = ds;
-    g.tens.base = db;
+    g.tens.iperm = dp + perm.size();
+    g.tens.slot_of = g.tens.iperm + iperm.size();
+    g.tens.base = g.tens.slot_of + slot_of.size();
     g.tens.fwt = dw;
     if (ctx->av) {  // P1 nodal functions at the tensor-ordered nodes (node artificial viscosity)
       const int N = r.order + 1;
