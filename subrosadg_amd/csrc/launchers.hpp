@@ -9,6 +9,7 @@
 #include "../../include/sdg.h"
 #include "dg_adjoint.hpp"
 #include "dg_kernels.hpp"
+#include "dg_line.hpp"
 #include "dg_mfma.hpp"
 #include "dg_quad.hpp"
 #include "dg_tensor.hpp"
@@ -23,6 +24,7 @@ using MonFn = void (*)(hipStream_t, const double*, int, double*, int*);
 using SrcFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, double*, const double*);
 using AdjFn = void (*)(hipStream_t, const Geo&, const Phys&, const StageArgs&, const AdjArgs&);
 using AvFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, double*);
+using LineFn = void (*)(hipStream_t, const Geo&, const Phys&, const LineRun&);
 using BlockFn = void (*)(hipStream_t, const Geo&, const Phys&, const double*, double*);
 
 struct Launchers {
@@ -48,6 +50,7 @@ struct Launchers {
   AvFn av_sensor = nullptr;
   // Navier-Stokes BR2 raw files: per boundary face the parent's volume gradient plus that face's lift
   BlockFn br2_blocks = nullptr;
+  LineFn line_run[2] = {nullptr, nullptr};  // lines, Euler: whole runs of small meshes (without / with AV)
   // discrete adjoint (Navier-Stokes, FP64: the dense matrix-core set, or the sum-factorised set on hexahedra)
   AdjFn adj_volume[2] = {nullptr, nullptr};  // BR1, BR2
   AdjFn adj_face = nullptr;
@@ -349,6 +352,19 @@ bool pickQuad(Launchers& l) {
     hipLaunchKernelGGL((quadTraceKernel<N>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, U, static_cast<double*>(Uf));
   };
   l.quad = true;
+  return true;
+}
+
+// Lines: the vector kernels, and the whole-run kernels of small Euler meshes
+template <int N>
+bool pickLine(bool mixed, Launchers& l) {
+  if (!pickValu<1, N, N, 2, 1>(mixed, l)) return false;
+  l.line_run[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const LineRun& a) {
+    hipLaunchKernelGGL((lineRunKernel<N, false>), dim3(1), dim3((g.E + 63) / 64 * 64), 0, st, g, ph, a);
+  };
+  l.line_run[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const LineRun& a) {
+    hipLaunchKernelGGL((lineRunKernel<N, true>), dim3(1), dim3((g.E + 63) / 64 * 64), 0, st, g, ph, a);
+  };
   return true;
 }
 

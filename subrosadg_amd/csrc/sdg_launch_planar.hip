@@ -6,11 +6,11 @@ namespace sdg {
 // 1-D: vector kernels (P+1 modes, P+1 Gauss points, two end-point faces)
 bool selectLine(int order, bool mixed, Launchers& l) {
   switch (order) {
-    case 1: return pickValu<1, 2, 2, 2, 1>(mixed, l);
-    case 2: return pickValu<1, 3, 3, 2, 1>(mixed, l);
-    case 3: return pickValu<1, 4, 4, 2, 1>(mixed, l);
-    case 4: return pickValu<1, 5, 5, 2, 1>(mixed, l);
-    case 5: return pickValu<1, 6, 6, 2, 1>(mixed, l);
+    case 1: return pickLine<2>(mixed, l);
+    case 2: return pickLine<3>(mixed, l);
+    case 3: return pickLine<4>(mixed, l);
+    case 4: return pickLine<5>(mixed, l);
+    case 5: return pickLine<6>(mixed, l);
     default: return false;
   }
 }

@@ -43,12 +43,12 @@ bool selectLaunchers(int type, int order, bool force_valu, bool mixed, Launchers
 }
 
 // 1-D tables and node/face maps of the sum-factorised kernels (hexahedra: dg_tensor.hpp,
-// quadrangles: dg_quad.hpp).
+// quadrangles: dg_quad.hpp, lines: dg_line.hpp).
 bool buildTensorTables(const sdg::RefElement& r, sdg::TensorOps& t, std::vector<short>& perm, std::vector<short>& iperm,
                        std::vector<short>& slot_of, std::vector<short>& base, std::vector<double>& fwt) {
-  const int N = r.order + 1, D = r.type == SDG_ELEM_HEXAHEDRON ? 3 : 2, NF = 2 * D;
-  const int NFQ = D == 3 ? N * N : N, NPT = N * NFQ;
-  if ((r.type != SDG_ELEM_HEXAHEDRON && r.type != SDG_ELEM_QUADRANGLE) || N > sdg::kTensorMaxN || r.nb != NPT ||
+  const int N = r.order + 1, D = r.dim, NF = 2 * D;
+  const int NFQ = D == 3 ? N * N : (D == 2 ? N : 1), NPT = N * NFQ;
+  if ((r.type != SDG_ELEM_HEXAHEDRON && r.type != SDG_ELEM_QUADRANGLE && r.type != SDG_ELEM_LINE) || N > sdg::kTensorMaxN || r.nb != NPT ||
       r.nq != NPT || r.nfq != NFQ)
     return false;
   std::vector<double> gx, gw;
@@ -292,6 +292,7 @@ struct sdg_ctx {
   hipGraphExec_t adjst_graph[2] = {nullptr, nullptr};
   double adjst_graph_dt[2] = {0.0, 0.0};
   bool use_graph = true;
+  bool line_run = false;  // small 1-D Euler mesh: a call of sdg_step is one launch (dg_line.hpp)
   float last_ms = 0.0f;
 
   bool ns() const { return prob.equation == SDG_EQ_COMPRESSIBLE_NS; }
@@ -479,6 +480,29 @@ void enqueueStep(sdg_ctx* ctx, double dt) {
 
 // Enqueue nsteps whole steps (each replayed from a captured graph) without waiting for them.
 int launchSteps(sdg_ctx* ctx, double dt, int nsteps) {
+  if (ctx->line_run && nsteps > 0) {
+    sdg::LineRun a{};
+    a.stages = ctx->stages();
+    for (int st = 0; st < a.stages; st++) {
+      double c[3];
+      ctx->rkCoefficients(st, c);
+      a.c0[st] = c[0];
+      a.c1[st] = c[1];
+      a.c2dt[st] = c[2] * dt;
+    }
+    a.U = ctx->U;
+    a.nodeav = ctx->nodeav;
+    a.rel = ctx->rel;
+    a.status = ctx->status;
+    for (int left = nsteps; left > 0; left -= a.nsteps) {
+      a.nsteps = std::min(left, sdg::kLineMaxSteps);
+      ctx->cur ^= (a.stages & a.nsteps) & 1;  // the trace buffer after stages x nsteps stages
+      a.Uf = ctx->Uf[ctx->cur];
+      ctx->launch.line_run[ctx->av ? 1 : 0](ctx->stream, ctx->geo, ctx->phys, a);
+    }
+    HIP_TRY(ctx, hipGetLastError());
+    return SDG_OK;
+  }
   for (int i = 0; i < nsteps; i++) {
     if (ctx->use_graph) {
       const int c = ctx->cur;
@@ -667,7 +691,12 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   // P2-P4 (FP64 or mixed), else the FP64 vector kernels
   const bool tensor_av = ctx->av && tensor && tensor_size;
   const bool av_vector = ctx->av && problem->equation == SDG_EQ_COMPRESSIBLE_NS && !tensor_av;
-  if (!selectLaunchers(r.type, r.order, force_vector || av_vector, mixed, ctx->launch,
+  // Tetrahedra P1, Navier-Stokes: a basis of 4 leaves most of a 16 x 16 tile empty, and on a small mesh
+  // the vector kernels' two launches a stage beat the matrix-core kernels' three (1296 elements: 41
+  // against 44 us a step; 2058 elements: 62 against 49)
+  const bool small_p1 = r.type == SDG_ELEM_TETRAHEDRON && r.order == 1 && mesh.elements <= 1536 &&
+                        problem->equation == SDG_EQ_COMPRESSIBLE_NS && problem->kernels == SDG_KERNELS_AUTO;
+  if (!selectLaunchers(r.type, r.order, force_vector || av_vector || small_p1, mixed, ctx->launch,
                        tensor && (!ctx->av || tensor_av))) {
     delete ctx;
     return fail(nullptr, SDG_E_UNSUPPORTED,
@@ -828,6 +857,11 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   ctx->Fb = Fb;
   Geo& g = ctx->geo;
   const bool sum_fact = ctx->launch.tensor || ctx->launch.quad;  // sum-factorised stage kernels
+  // Small 1-D Euler meshes run whole calls of sdg_step in one workgroup, an element a thread.
+  ctx->line_run = r.type == SDG_ELEM_LINE && !ctx->ns() && !mixed && !curved && problem->kernels == SDG_KERNELS_AUTO &&
+                  problem->launch == SDG_LAUNCH_GRAPH && problem->source_term == SDG_SOURCE_NONE &&
+                  E <= sdg::kLineMaxElements && ctx->launch.line_run[ctx->av ? 1 : 0];
+  const bool tensor_tables = sum_fact || ctx->line_run;
   if (!curved) {  // straight faces: normal and area factor once per face, and per element face
     std::vector<double> fgeo(static_cast<size_t>(ctx->F) * (D + 1));
     for (int64_t f = 0; f < ctx->F; f++) {
@@ -838,7 +872,7 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     if (upload(ctx, fgeo, &df) || upload(ctx, r.fweight, &dw)) return bail(SDG_E_NOMEM);
     g.fgeo = df;
     g.fwl = dw;
-    if (sum_fact) {
+    if (tensor_tables) {
       std::vector<double> egeo(static_cast<size_t>(E) * r.nf * (D + 1));
       for (size_t o = 0; o < static_cast<size_t>(E) * r.nf; o++) {
         double* eg = &egeo[o * (D + 1)];
@@ -1057,7 +1091,7 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     g.op.lift = pl;
     g.op.rinterp = pi;
   }
-  if (sum_fact) {
+  if (tensor_tables) {
     std::vector<short> perm, iperm, slot_of, base;
     std::vector<double> fwt;
     if (!buildTensorTables(r, g.tens, perm, iperm, slot_of, base, fwt))
@@ -1077,7 +1111,7 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
       std::vector<double> gx, gw, nodt(static_cast<size_t>(nb) * r.nvert);
       sdg::gaussLegendre(N, gx, gw);
       for (int q = 0; q < nb; q++) {
-        const double xi[3] = {gx[q % N], gx[(q / N) % N], D == 3 ? gx[q / (N * N)] : 0.0};
+        const double xi[3] = {gx[q % N], D > 1 ? gx[(q / N) % N] : 0.0, D == 3 ? gx[q / (N * N)] : 0.0};
         sdg::nodalValues(r, xi, &nodt[static_cast<size_t>(q) * r.nvert]);
       }
       double* dn;
