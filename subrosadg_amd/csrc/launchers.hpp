@@ -12,6 +12,7 @@
 #include "dg_line.hpp"
 #include "dg_mfma.hpp"
 #include "dg_quad.hpp"
+#include "dg_quad_adjoint.hpp"
 #include "dg_tensor.hpp"
 #include "dg_tensor_adjoint.hpp"
 
@@ -323,8 +324,8 @@ bool selectTensorAvT(int order, Launchers& l) {
     default: return false;
   }
 }
-// Quadrangles, FP64: the sum-factorised stage kernels replace those of every stage (the adjoint kernels
-// stay). 256^2 P3 Euler with artificial viscosity: 95 us of kernels a stage, 260 us on the matrix-core
+// Quadrangles, FP64: the sum-factorised stage kernels replace those of every stage, and their
+// transpose the adjoint kernels where the size has an adjoint. 256^2 P3 Euler with artificial viscosity: 95 us of kernels a stage, 260 us on the matrix-core
 // kernels; 48^2 P3 Navier-Stokes: 14.3 us and 28 us; 32^2 P2 Euler: 7.1 us and 8.5 us on the vector kernel.
 template <int N>
 bool pickQuad(Launchers& l) {
@@ -351,6 +352,23 @@ bool pickQuad(Launchers& l) {
   l.trace = [](hipStream_t st, const Geo& g, const double* U, void* Uf, const MixRef&) {
     hipLaunchKernelGGL((quadTraceKernel<N>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, U, static_cast<double*>(Uf));
   };
+  if (l.adj_face) {  // P3..P5: the transpose of these kernels (the face kernel is the generic one)
+    l.adj_volume[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
+      hipLaunchKernelGGL((quadAdjVolume<N, 1>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, ph, a, j);
+    };
+    l.adj_volume[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
+      hipLaunchKernelGGL((quadAdjVolume<N, 2>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, ph, a, j);
+    };
+    l.adj_lift[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
+      hipLaunchKernelGGL((quadAdjLift<N, 1>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, ph, a, j);
+    };
+    l.adj_lift[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
+      hipLaunchKernelGGL((quadAdjLift<N, 2>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, ph, a, j);
+    };
+    l.adj_gather = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
+      hipLaunchKernelGGL((quadAdjGather<N>), dim3(blocksFor(g.E, EPB)), dim3(64), 0, st, g, ph, a, j);
+    };
+  }
   l.quad = true;
   return true;
 }

@@ -692,8 +692,8 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   const bool tensor_av = ctx->av && tensor && tensor_size;
   const bool av_vector = ctx->av && problem->equation == SDG_EQ_COMPRESSIBLE_NS && !tensor_av;
   // Tetrahedra P1, Navier-Stokes: a basis of 4 leaves most of a 16 x 16 tile empty, and on a small mesh
-  // the vector kernels' two launches a stage beat the matrix-core kernels' three (1296 elements: 41
-  // against 44 us a step; 2058 elements: 62 against 49)
+  // the vector kernels' two launches a stage beat the matrix-core kernels' three (1296 elements: 79
+  // against 89 us a step; 2058 elements: 124 against 98)
   const bool small_p1 = r.type == SDG_ELEM_TETRAHEDRON && r.order == 1 && mesh.elements <= 1536 &&
                         problem->equation == SDG_EQ_COMPRESSIBLE_NS && problem->kernels == SDG_KERNELS_AUTO;
   if (!selectLaunchers(r.type, r.order, force_vector || av_vector || small_p1, mixed, ctx->launch,
@@ -981,9 +981,8 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
     g.ntag = dtag;
     g.nodeav = ctx->nodeav;
   }
-  // padded operators of the matrix-core kernels (the sum-factorised quadrangles use them in the adjoint,
-  // on periodic Navier-Stokes meshes)
-  if (ctx->launch.mfma && (!ctx->launch.quad || (ctx->ns() && Fb == 0))) {
+  // padded operators of the matrix-core kernels
+  if (ctx->launch.mfma && !ctx->launch.quad) {
     const int nfq_ = nfq;
     auto V = [&](int q, int b) { return r.V[static_cast<size_t>(q) * nb + b]; };
     auto Vfv = [&](int sl, int b) { return r.Vf[static_cast<size_t>(sl) * nb + b]; };
