@@ -92,14 +92,16 @@ enum sdg_boundary {
   SDG_BC_PERIODIC = 6
 };
 
-/* Kernel family of a single-problem context. AUTO: sum-factorised Navier-Stokes kernels on
- * hexahedra P2-P4, dense matrix-core kernels on the other matrix-core sizes (quadrangles P3-P5,
- * hexahedra P2-P4 Euler), vector kernels elsewhere. DENSE keeps the dense matrix-core kernels on
- * hexahedra; VECTOR runs the vector kernels for every size (FP64 only). All evaluate the same
+/* Kernel family of a single-problem context. AUTO: sum-factorised kernels on hexahedra P2-P4
+ * (Navier-Stokes) and quadrangles P1-P5 (FP64), dense matrix-core kernels on the other matrix-core
+ * sizes (quadrangles P3-P5 in mixed precision, hexahedra P2-P4 Euler, triangles and tetrahedra in
+ * FP64), vector kernels elsewhere. DENSE keeps the dense matrix-core kernels where a size has them;
+ * VECTOR runs the vector kernels for every size (FP64 only). All evaluate the same
  * operator; the choice exists to compare them. */
 enum sdg_kernels { SDG_KERNELS_AUTO = 0, SDG_KERNELS_DENSE = 1, SDG_KERNELS_VECTOR = 2 };
 /* GRAPH: each sdg_step call replays whole steps from captured hipGraphs; EAGER: every kernel is
- * launched on the stream as it comes (same kernels, same results). */
+ * launched on the stream as it comes (same kernels, same results; on 1-D Euler meshes of up to 512
+ * elements GRAPH runs a call's steps in one launch, equal to rounding). */
 enum sdg_launch { SDG_LAUNCH_GRAPH = 0, SDG_LAUNCH_EAGER = 1 };
 
 /* Runtime copy of the reference's compile-time SimulationControl
