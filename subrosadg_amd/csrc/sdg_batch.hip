@@ -88,13 +88,16 @@ struct Args {
 };
 
 constexpr int kMaxNfq = 5;
+// workgroups of a variant kernel that its registers let a CU hold
+constexpr int residentOf(int flux) { return flux == SDG_FLUX_EXACT ? 3 : 4; }
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
 // Elements per panel: as many as the point phase (one thread per volume point or face point) takes in
-// one pass of the workgroup (one element more costs a second pass for a few points: 48 problems, 50
-// steps, mixed precision 42.6 -> 37.2 ms; FP64 panels are bounded by LDS, 44.1 ms either way), within an LDS budget for the panel (state, volume flux, face flux) so that
-// several workgroups share a CU.
+// one pass of the workgroup (one element more costs a second pass for a few points: 48 problems of 8^2
+// to 96^2 cells, Lax-Friedrichs, 828 -> 725 us a step in mixed precision and 775 -> 764 us in FP64, whose
+// P3 and P4 panels are bounded by LDS), within an LDS budget for the panel (state, volume flux, face flux)
+// so that several workgroups share a CU.
 template <typename TC, int NB, int NQ, int NF, int NFQ>
 struct Shape {
   static constexpr int NAQ = NF * NFQ;
@@ -310,7 +313,7 @@ __device__ __forceinline__ void eulerTile(const Args<TC>& a, const VariantDev& v
       for (int v = 0; v < NV; v++) {
         const int64_t gi = vd.u_base + (e * NV + v) * NB + i;
         uo[v] = a.U[gi];
-        uno[v] = a.c0 != 0.0 ? a.Un[gi] : 0.0;
+        uno[v] = a.Un[gi];
       }
       TC r[NV] = {}, hs[NV] = {};
 #pragma unroll 4
@@ -377,10 +380,15 @@ constexpr int epbOf(int code) {
 // One RK stage of one variant's elements (all problems): a persistent grid striding over that
 // variant's work items [begin, end). Each variant has its own kernel, so that its registers and LDS
 // are sized for its element type and order alone; the variants of a stage run concurrently (graph
-// branches).
+// branches). Bound to 128 registers, four workgroups a CU, which spills at most 32 bytes a lane (the exact
+// Riemann solver would spill up to 120 and gets 168, three workgroups): quadrangles P4, FP64,
+// Lax-Friedrichs, took 130 and with a grid of four a CU of which three were resident 716 us a step for 24
+// problems of 48^2 cells, 515 us now; the variants further above gain too, with HLLC 705 -> 536 us, and
+// triangles P3 in mixed precision 447 -> 318 us.
 template <typename TC, int FLUX, int CODE, int NB, int NQ, int NF, int NFQ>
-__global__ __launch_bounds__(kThreads) void batchVariantKernel(Args<TC> a, int begin, int end) {
+__global__ __launch_bounds__(kThreads, residentOf(FLUX)) void batchVariantKernel(Args<TC> a, int begin, int end) {
   using S = Shape<TC, NB, NQ, NF, NFQ>;
+  static_assert(residentOf(FLUX) * (S::LDS_ELEMS + S::TAB_ELEMS) * sizeof(TC) <= 160 * 1024, "LDS of the resident workgroups");
   __shared__ TC smem[S::LDS_ELEMS];
   __shared__ TC tab[S::TAB_ELEMS];
   const VariantDev& vd = a.var[CODE];
@@ -536,7 +544,7 @@ struct sdg_batch {
   sdg::batch::WorkItem* ditems = nullptr;
   int ditems_cap = 0;
   std::vector<sdg::batch::WorkItem> items;
-  int chunk[sdg::batch::kVariants] = {1, 1, 1, 1, 1, 1, 1, 1};  // work-item size in tiles
+  int chunk[sdg::batch::kVariants] = {};  // work-item size in tiles; 0: chunkFor
   int vgrid[sdg::batch::kVariants] = {};                         // persistent grid per variant kernel
   int ibeg[sdg::batch::kVariants] = {}, iend[sdg::batch::kVariants] = {};  // work items per variant
   // the variants of a stage run on their own streams, forked from and joined back into `stream`
@@ -631,6 +639,12 @@ int stagesOf(const sdg_batch* b) {
   return b->prob.time_integration == SDG_RK_FORWARD_EULER ? 1 : (b->prob.time_integration == SDG_RK_HEUN2 ? 2 : 3);
 }
 
+// Tiles per work item: one while every tile finds a workgroup of the grid, else two (a tile of its own
+// item costs 4 % more than one of two, 24 problems of 48^2 quadrangles P4 534 and 515 us a step). With
+// four for every size small batches ran up to four tiles in a row on a card with idle CUs: one problem of
+// 64^2 cells P2 118 -> 68 us a step, 48 problems of 8^2 to 24^2 cells P1-P4 320 -> 173 us.
+int chunkFor(int64_t tiles, int grid) { return tiles <= grid ? 1 : 2; }
+
 // work items: per variant, chunks of chunk[v] tiles
 int buildItems(sdg_batch* b, const int* only = nullptr) {
   b->items.clear();
@@ -639,6 +653,7 @@ int buildItems(sdg_batch* b, const int* only = nullptr) {
     b->ibeg[v] = b->iend[v] = static_cast<int>(b->items.size());
     if (!V.used || (only && v != *only)) continue;
     const int epb = b->mixed ? sdg::batch::epbOf<float>(v) : sdg::batch::epbOf<double>(v);
+    if (b->chunk[v] == 0) b->chunk[v] = chunkFor((V.E + epb - 1) / epb, b->vgrid[v]);
     const int64_t step = static_cast<int64_t>(b->chunk[v]) * epb;
     for (int64_t f = 0; f < V.E; f += step) b->items.push_back({v, static_cast<int>(std::min<int64_t>(step, V.E - f)), f});
     b->iend[v] = static_cast<int>(b->items.size());
@@ -1011,9 +1026,15 @@ int sdg_batch_create(const sdg_problem_desc* problem, const sdg_mesh* const* mes
   b->has_state.assign(count, 0);
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  for (int v = 0; v < sdg::batch::kVariants; v++) {
-    b->chunk[v] = 4;
-    b->vgrid[v] = cus * 4;
+  for (int v = 0; v < sdg::batch::kVariants; v++) {  // the workgroups that are resident at a time
+    const int flux = b->prob.convective_flux;
+    const void* kernel = b->mixed ? reinterpret_cast<const void*>(sdg::batch::variantKernel<float>(flux, v))
+                                  : reinterpret_cast<const void*>(sdg::batch::variantKernel<double>(flux, v));
+    int per_cu = 0;
+    if (!b->var[v].used || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, sdg::batch::kThreads, 0) != hipSuccess ||
+        per_cu < 1)
+      per_cu = sdg::batch::residentOf(flux);
+    b->vgrid[v] = cus * per_cu;
   }
   if (buildItems(b)) return bail(SDG_E_DEVICE);
   *out = b;

@@ -243,3 +243,26 @@ def test_c3_workload_48_uneven_problems():
     print(f"  mixed vs FP64 L2 deviation: max {devs[k]:.3e} (problem {k}: n={specs[k][0]}, P{specs[k][1]}), "
           f"median {float(np.median(devs)):.3e}", flush=True)
     assert max(devs) <= 1e-6, devs
+
+
+@pytest.mark.parametrize("flux", [L.FLUX_HLLC, L.FLUX_ROE])
+@pytest.mark.parametrize("n,tiles_per_item", [(1, 1), (40, 1), (170, 2)])
+def test_work_items_of_one_and_two_tiles(n, tiles_per_item, flux):
+    """Triangles P1 below and above as many tiles as resident workgroups: 3 steps of one problem against
+    the single-problem solver (two FP64 evaluations of one scheme)."""
+    mesh = L.Mesh.split(1, (max(n, 2), n + 1), (0.0, 0.0), (1.0, 1.0), 1.0, 7)
+    prob = L.problem_desc(cp=3.5, cv=2.5, equation=L.EQ_EULER, convective_flux=flux)
+    x = mesh.field("quad_coord").reshape(mesh.E, mesh.nq, 2)
+    prim = np.zeros((mesh.E, mesh.nq, 4))
+    prim[..., 0] = 1.0 + 0.2 * np.sin(2 * np.pi * x[..., 0])
+    prim[..., 1], prim[..., 2] = 0.3, 0.1 * np.cos(2 * np.pi * x[..., 1])
+    prim[..., 3] = 1.0 + 0.1 * np.cos(2 * np.pi * x[..., 0])
+    b, s = L.Batch(prob, [mesh]), L.Solver(prob, mesh)
+    assert b.config()[0].max() == tiles_per_item
+    s.set_initial_primitive(prim)
+    b.set_state(0, s.get_state())
+    dt = s.compute_dt(0.1)
+    s.step(dt, 3)
+    b.step([dt], 3)
+    u = s.get_state()
+    assert P.parity_error(b.get_state(0).reshape(u.shape), u, u, 2) <= 1e-12
