@@ -193,14 +193,20 @@ __device__ __forceinline__ double faceStateVjpDir(const Phys& ph, const double* 
   return s;
 }
 
+// Workgroup of the adjoint kernels: their tallest operator has NQ D rows (the transposed gradient).
+// With as many wavefronts as the forward operators have row tiles, a step of the adjoint of 6^2
+// quadrangles took 201 us at P3 and 233 at P4, now 188 and 220; 64^2 P5 776 and now 740.
+template <int D, int NB, int NQ, int NAQ>
+using AdjShape = MfmaShape<NB, NQ * D, NAQ>;
+
 // ---- kernel 1: volume part ----------------------------------------------------------------------
 template <int D, int NB, int NQ, int NF, int NFQ, int VISC>
-__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjVolumeMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
+__global__ __launch_bounds__((AdjShape<D, NB, NQ, NF * NFQ>::NT)) void nsAdjVolumeMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
   constexpr int NV = LD::NV, NG = LD::NG, EPB = LD::EPB, NAQ = LD::NAQ;
   constexpr int NBk = LD::NBk, NBm = LD::NBm, NQm = LD::NQm, NQk = r4(NQ), NAQm = LD::NAQm;
   constexpr int NBr = LD::NBr, NDQm = r16(NQ * D);
-  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
+  constexpr int NT = AdjShape<D, NB, NQ, NF * NFQ>::NT, STEP = AdjShape<D, NB, NQ, NF * NFQ>::STEP;
   constexpr int AJV = LD::AJ > 2 * NQm * 16 ? LD::AJ : 2 * NQm * 16;  // grad u_q and grad-bar_q
   static_assert(2 * NBr >= NQm, "u-bar_q reuses the lifting work area");
   __shared__ double sUq[NQm * 16];
@@ -211,7 +217,7 @@ __global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjVolume
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
   const int e0 = blockIdx.x * EPB;
-  gradLift<double, D, NB, NQ, NF, NFQ, VISC>(g, ph, a, e0, sUq, sAJ, sRR);
+  gradLift<double, D, NB, NQ, NF, NFQ, VISC, AdjShape<D, NB, NQ, NF * NFQ>::WAVES>(g, ph, a, e0, sUq, sAJ, sRR);
   double* sGq = sAJ;
   double* sLam = sRR;
   double* sMu = sRR + NBr * 16;
@@ -409,12 +415,12 @@ __global__ __launch_bounds__(kThreads) void nsAdjFaceRevKernel(Geo g, Phys ph, S
 
 // ---- kernel 3: lifting terms --------------------------------------------------------------------
 template <int D, int NB, int NQ, int NF, int NFQ, int VISC>
-__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjLiftMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
+__global__ __launch_bounds__((AdjShape<D, NB, NQ, NF * NFQ>::NT)) void nsAdjLiftMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
   constexpr int NV = LD::NV, NG = LD::NG, EPB = LD::EPB, NAQ = LD::NAQ;
   constexpr int NBk = LD::NBk, NBm = LD::NBm, NQm = LD::NQm, NQk = r4(NQ), NAQk = LD::NAQk, NAQm = LD::NAQm;
   constexpr int NBr = LD::NBr, NDQm = r16(NQ * D);
-  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
+  constexpr int NT = AdjShape<D, NB, NQ, NF * NFQ>::NT, STEP = AdjShape<D, NB, NQ, NF * NFQ>::STEP;
   __shared__ double sRt[NBr * 16];
   __shared__ double sRw[NBr * 16];
   __shared__ double sGb[NAQm * 16];
@@ -537,10 +543,10 @@ __global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjLiftMf
 
 // ---- kernel 4: gather the trace adjoints and apply Vf^T ---------------------------------------
 template <int D, int NB, int NQ, int NF, int NFQ>
-__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsAdjGatherMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
+__global__ __launch_bounds__((AdjShape<D, NB, NQ, NF * NFQ>::NT)) void nsAdjGatherMfma(Geo g, Phys ph, StageArgs a, AdjArgs j) {
   constexpr int NV = D + 2, NAQ = NF * NFQ, EPB = 16 / NV;
   constexpr int NBm = r16(NB), NAQk = r4(NAQ);
-  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
+  constexpr int NT = AdjShape<D, NB, NQ, NF * NFQ>::NT, STEP = AdjShape<D, NB, NQ, NF * NFQ>::STEP;
   __shared__ double sUf[NAQk * 16];
   const MOps& op = g.op;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

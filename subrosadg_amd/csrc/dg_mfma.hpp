@@ -72,13 +72,16 @@ __device__ __forceinline__ void tileStore(const acc_t<TC>& acc, TC* Y, int m0, i
 
 // Workgroup of a matrix-core kernel: one wavefront per 16-row tile of its tallest operator, at most
 // four. A tile is one wavefront's chain of matrix instructions, so further wavefronts only wait at
-// the barriers, and at one tile (quadrangles P3) the barriers cost nothing at all.
+// the barriers, and at one tile (quadrangles P3) the barriers cost nothing at all. On a grid of few
+// workgroups (kWideGrid) the gradient and residual kernels take four nevertheless: CUs are idle there,
+// and the pointwise phases and the panel loads run in fewer rounds one after the other.
 template <int NB, int NQ, int NAQ>
 struct MfmaShape {
   static constexpr int TILES = r16(NB > NQ ? (NB > NAQ ? NB : NAQ) : (NQ > NAQ ? NQ : NAQ)) / 16;
   static constexpr int WAVES = TILES < 4 ? TILES : 4;
   static constexpr int NT = 64 * WAVES, STEP = 16 * WAVES;
 };
+constexpr int kWideWaves = 4;
 
 template <int NT, typename TC>
 __device__ __forceinline__ void zeroLds(TC* p, int n, int tid) {
@@ -153,13 +156,13 @@ __device__ __forceinline__ void addSource(const Geo& g, const StageArgs& a, int 
   __syncthreads();
 }
 
-template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int EPB>
+template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int EPB, int WAVES>
 __device__ __forceinline__ void mfmaStageTail(const Geo& g, const StageArgs& a, int e0, TC* sR, TC* sU,
                                               double* sRed) {
   constexpr int NV = D + 2, NAQ = NF * NFQ;
   constexpr int NBk = r4(NB), NBm = r16(NB), NQm = r16(NQ), NAQm = r16(NAQ);
   constexpr bool MIX = sizeof(TC) == 4;
-  constexpr int STEP = MfmaShape<NB, NQ, NAQ>::STEP, WAVES = MfmaShape<NB, NQ, NAQ>::WAVES;
+  constexpr int STEP = 16 * WAVES;
   const MOpsT<TC>& op = opsOf<TC>(g);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, rr = lane >> 4;
@@ -426,7 +429,7 @@ __global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void eulerStageM
     }
     return;
   }
-  mfmaStageTail<TC, D, NB, NQ, NF, NFQ, EPB>(g, a, e0, sR, sU, sRed);
+  mfmaStageTail<TC, D, NB, NQ, NF, NFQ, EPB, MfmaShape<NB, NQ, NAQ>::WAVES>(g, a, e0, sR, sU, sRed);
 }
 
 // ---- Navier-Stokes kernel 1 (MFMA): gradient lifting + volume flux -------------------------------
@@ -452,7 +455,7 @@ struct GradLds {
 //   Gf (HBM)            lifted gradient traces at the element's face points, and, if a.Wout is
 //                       set, the lifted total-gradient coefficients;
 // sRR is free again. Ends with a barrier.
-template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int VISC>
+template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int VISC, int WAVES>
 __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const StageArgs& a, int e0, TC* sUq, TC* sAJ,
                                          TC* sRR) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
@@ -460,7 +463,7 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   constexpr int NV = LD::NV, NG = LD::NG, NAQ = LD::NAQ, EPB = LD::EPB;
   constexpr int NBk = LD::NBk, NBm = LD::NBm, NQm = LD::NQm, NAQk = LD::NAQk, NAQm = LD::NAQm, NDQk = LD::NDQk;
   constexpr int NBr = LD::NBr, AJ = LD::AJ;
-  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
+  constexpr int NT = 64 * WAVES, STEP = 16 * WAVES;
   TC* sU = sRR;
   TC* sA = sAJ;
   TC* sJ = sAJ + NAQk * 16;
@@ -598,18 +601,18 @@ __device__ __forceinline__ void gradLift(const Geo& g, const Phys& ph, const Sta
   __syncthreads();
 }
 
-template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int VISC>
-__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsGradMfma(Geo g, Phys ph, StageArgs a) {
+template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int VISC, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void nsGradMfma(Geo g, Phys ph, StageArgs a) {
   using LD = GradLds<D, NB, NQ, NF, NFQ>;
   constexpr int NV = LD::NV, NG = LD::NG, EPB = LD::EPB;
-  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT;
+  constexpr int NT = 64 * WAVES;
   __shared__ TC sUq[LD::NQm * 16];      // state at volume points
   __shared__ TC sAJ[LD::AJ];            // face terms A | J ([slot][le*NG + r]); later the gradient at points
   __shared__ TC sRR[2 * LD::NBr * 16];  // state panel; then R_w | R_t
   if (a.status && a.status[0]) return;
   const int tid = threadIdx.x;
   const int e0 = blockIdx.x * EPB;
-  gradLift<TC, D, NB, NQ, NF, NFQ, VISC>(g, ph, a, e0, sUq, sAJ, sRR);
+  gradLift<TC, D, NB, NQ, NF, NFQ, VISC, WAVES>(g, ph, a, e0, sUq, sAJ, sRR);
   const TC* sGq = sAJ;
   // volume flux (F_c - F_v)^T (J^T)^-1 |J| w at the points -> HBM Fv[e][(q D + b)][v]; the weak
   // divergence F Phi_grad is taken in nsResidualMfma, which packs three elements per 16 columns
@@ -760,15 +763,15 @@ __global__ __launch_bounds__(kThreads) void nsFaceFluxKernel(Geo g, Phys ph, Sta
 // ---- Navier-Stokes residual + update + next traces (MFMA), after nsFaceFluxKernel ---------------
 // calculateResidual + updateBasisFunctionCoefficient (SpatialDiscrete.cpp:1016-1032,
 // TimeIntegration.cpp:181-198)
-template <typename TC, int D, int NB, int NQ, int NF, int NFQ>
-__global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsResidualMfma(Geo g, Phys ph, StageArgs a) {
+template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void nsResidualMfma(Geo g, Phys ph, StageArgs a) {
   const MOpsT<TC>& op = opsOf<TC>(g);
   constexpr int NV = D + 2, NAQ = NF * NFQ;
   constexpr int EPB = 16 / NV;
   constexpr int NBk = r4(NB), NBm = r16(NB), NAQk = r4(NAQ);
   constexpr int NBr = NBk > NBm ? NBk : NBm;
   constexpr int NDQ = NQ * D, NDQk = r4(NDQ);
-  constexpr int NT = MfmaShape<NB, NQ, NF * NFQ>::NT, STEP = MfmaShape<NB, NQ, NF * NFQ>::STEP;
+  constexpr int NT = 64 * WAVES, STEP = 16 * WAVES;
   __shared__ TC sU[NBr * 16];
   __shared__ TC sH[NAQk * 16];
   __shared__ TC sF[NDQk * 16];
@@ -814,7 +817,7 @@ __global__ __launch_bounds__((MfmaShape<NB, NQ, NF * NFQ>::NT)) void nsResidualM
     }
     return;
   }
-  mfmaStageTail<TC, D, NB, NQ, NF, NFQ, EPB>(g, a, e0, sR, sU, sRed);
+  mfmaStageTail<TC, D, NB, NQ, NF, NFQ, EPB, WAVES>(g, a, e0, sR, sU, sRed);
 }
 
 // Traces at the element's own face points from the state in HBM, with the same operands and

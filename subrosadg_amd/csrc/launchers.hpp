@@ -61,6 +61,35 @@ struct Launchers {
 
 inline int blocksFor(int E, int epb) { return (E + epb - 1) / epb; }
 
+// Grids of at most this many workgroups take kWideWaves wavefronts each in the gradient and residual
+// kernels. Microseconds a launch at 507 to 1024, 2025 to 2048 and 12800 workgroups, with the tile count's
+// wavefronts and with four: quadrangles P3 FP64 gradient 12.8 and 12.0, 17.7 and 20.2, 52.5 and 69.5.
+constexpr int kWideGrid = 1024;
+// In FP64 the residual kernel takes four for any grid where the flux panel it stages has 24 rows or more:
+// quadrangles P3 10.3 and 7.9 us at 256 workgroups, 32.0 and 30.4 at 6400; tetrahedra P2 22.7 and 20.0 at
+// 3456. Below (triangles P1, P2, tetrahedra P1) and in mixed precision it loses on large grids: triangles
+// P2 12.8 and 15.5 us at 5000 workgroups, quadrangles P4 mixed 35.3 and 40.8 at 6400.
+constexpr int kWideRows = 24;
+
+template <typename TC, int D, int NB, int NQ, int NF, int NFQ, int VISC>
+void launchGradMfma(hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
+  constexpr int W = MfmaShape<NB, NQ, NF * NFQ>::WAVES;
+  const int grid = blocksFor(g.E, 16 / ((D + 2) * D));
+  if (W < kWideWaves && grid <= kWideGrid)
+    hipLaunchKernelGGL((nsGradMfma<TC, D, NB, NQ, NF, NFQ, VISC, kWideWaves>), dim3(grid), dim3(64 * kWideWaves), 0, st, g, ph, a);
+  else
+    hipLaunchKernelGGL((nsGradMfma<TC, D, NB, NQ, NF, NFQ, VISC, W>), dim3(grid), dim3(64 * W), 0, st, g, ph, a);
+}
+template <typename TC, int D, int NB, int NQ, int NF, int NFQ>
+void launchResidualMfma(hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
+  constexpr int W = sizeof(TC) == 8 && NQ * D >= kWideRows ? kWideWaves : MfmaShape<NB, NQ, NF * NFQ>::WAVES;
+  const int grid = blocksFor(g.E, 16 / (D + 2));
+  if (W < kWideWaves && grid <= kWideGrid)
+    hipLaunchKernelGGL((nsResidualMfma<TC, D, NB, NQ, NF, NFQ, kWideWaves>), dim3(grid), dim3(64 * kWideWaves), 0, st, g, ph, a);
+  else
+    hipLaunchKernelGGL((nsResidualMfma<TC, D, NB, NQ, NF, NFQ, W>), dim3(grid), dim3(64 * W), 0, st, g, ph, a);
+}
+
 // VALU kernels: any size; MFMA kernels: bases that fill 16x16 tiles. TC is the contraction type of
 // the matrix-core kernels: double (FP64 mode) or float (mixed-precision mode).
 template <int D, int NB, int NQ, int NF, int NFQ, bool MFMA, typename TC = double, bool ADJOINT = true>
@@ -77,31 +106,26 @@ Launchers makeLaunchers() {
                          dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
     };
     l.ns_grad_br1 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((nsGradMfma<TC, D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)), dim3(MfmaShape<NB, NQ, NF * NFQ>::NT),
-                         0, st, g, ph, a);
+      launchGradMfma<TC, D, NB, NQ, NF, NFQ, 1>(st, g, ph, a);
     };
     l.ns_grad_br2 = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((nsGradMfma<TC, D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)), dim3(MfmaShape<NB, NQ, NF * NFQ>::NT),
-                         0, st, g, ph, a);
+      launchGradMfma<TC, D, NB, NQ, NF, NFQ, 2>(st, g, ph, a);
     };
     l.ns_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
       hipLaunchKernelGGL((nsFaceFluxKernel<TC, D, NF, NFQ>), dim3(blocksFor((g.F + g.Fb) * NFQ, kThreads)),
                          dim3(kThreads), 0, st, g, ph, a);
     };
     l.ns_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-      hipLaunchKernelGGL((nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)), dim3(MfmaShape<NB, NQ, NF * NFQ>::NT),
-                         0, st, g, ph, a);
+      launchResidualMfma<TC, D, NB, NQ, NF, NFQ>(st, g, ph, a);
     };
     {  // Euler with artificial viscosity: volume gradient, AV fluxes (both precision modes)
       l.av_grad = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
-        hipLaunchKernelGGL((nsGradMfma<TC, D, NB, NQ, NF, NFQ, 0>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
+        launchGradMfma<TC, D, NB, NQ, NF, NFQ, 0>(st, g, ph, a);
       };
       l.av_flux = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a) {
         hipLaunchKernelGGL((nsFaceFluxKernel<TC, D, NF, NFQ, false, true>),
                            dim3(blocksFor((g.F + g.Fb) * NFQ, kThreads)), dim3(kThreads), 0, st, g, ph, a);
-        hipLaunchKernelGGL((nsResidualMfma<TC, D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a);
+        launchResidualMfma<TC, D, NB, NQ, NF, NFQ>(st, g, ph, a);
       };
       l.av_sensor = [](hipStream_t st, const Geo& g, const Phys& ph, const double* U, double* node) {
         hipLaunchKernelGGL((avSensorKernel<D, NB, NQ>), dim3(blocksFor(g.E, kThreads)), dim3(kThreads),
@@ -111,11 +135,11 @@ Launchers makeLaunchers() {
     if constexpr (ADJOINT && sizeof(TC) == 8) {
       l.adj_volume[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
         hipLaunchKernelGGL((nsAdjVolumeMfma<D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
+                           dim3(AdjShape<D, NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_volume[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
         hipLaunchKernelGGL((nsAdjVolumeMfma<D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
+                           dim3(AdjShape<D, NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_face = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
         if (ph.flux <= SDG_FLUX_ROE)  // reverse mode, one thread per face point
@@ -128,15 +152,15 @@ Launchers makeLaunchers() {
       };
       l.adj_lift[0] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
         hipLaunchKernelGGL((nsAdjLiftMfma<D, NB, NQ, NF, NFQ, 1>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
+                           dim3(AdjShape<D, NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_lift[1] = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
         hipLaunchKernelGGL((nsAdjLiftMfma<D, NB, NQ, NF, NFQ, 2>), dim3(blocksFor(g.E, EPB_G)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
+                           dim3(AdjShape<D, NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
       l.adj_gather = [](hipStream_t st, const Geo& g, const Phys& ph, const StageArgs& a, const AdjArgs& j) {
         hipLaunchKernelGGL((nsAdjGatherMfma<D, NB, NQ, NF, NFQ>), dim3(blocksFor(g.E, EPB_S)),
-                           dim3(MfmaShape<NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
+                           dim3(AdjShape<D, NB, NQ, NF * NFQ>::NT), 0, st, g, ph, a, j);
       };
     }
   } else {

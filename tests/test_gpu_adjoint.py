@@ -22,12 +22,42 @@ CASES = [
     ("tgv-hex-p4-lf-br1", lambda: P.ns_tgv(n=2, order=4, flux=L.FLUX_LAX_FRIEDRICHS, visc=L.VISC_BR1)),
     ("tgv-hex-p4-hllc-br2", lambda: P.ns_tgv(n=2, order=4)),
     ("tgv-hex-p3-roe-br2-dense", lambda: _dense(P.ns_tgv(n=2, order=3, flux=L.FLUX_ROE))),
+    # dense matrix-core kernels in workgroups of fewer than four wavefronts
+    ("shear-quad-p3-roe-br2-dense", lambda: _dense(P.ns_shear(n=4, order=3, perturb=True))),
+    ("shear-quad-p3-hllc-br1-dense", lambda: _dense(P.ns_shear(n=3, order=3, flux=L.FLUX_HLLC, visc=L.VISC_BR1, perturb=True))),
+    ("shear-quad-p4-lf-br2-dense", lambda: _dense(P.ns_shear(n=3, order=4, flux=L.FLUX_LAX_FRIEDRICHS, perturb=True))),
+    # sum-factorised quadrangles whose last wavefront is partly filled (4, 2 and 1 elements each), sheared cells
+    ("sheared-quad-p3-hllc-br2", lambda: _sheared(3, 3, L.VISC_BR2)),
+    ("sheared-quad-p3-hllc-br1", lambda: _sheared(3, 3, L.VISC_BR1)),
+    ("sheared-quad-p4-hllc-br2", lambda: _sheared(3, 4, L.VISC_BR2)),
+    ("sheared-quad-p4-hllc-br1", lambda: _sheared(3, 4, L.VISC_BR1)),
+    ("sheared-quad-p5-hllc-br2", lambda: _sheared(3, 5, L.VISC_BR2)),
+    ("sheared-quad-p5-hllc-br1", lambda: _sheared(3, 5, L.VISC_BR1)),
+]
+# the product of this case is 1.2e-3 of the sum of the absolute products, so that the central difference's
+# rounding alone is 2e-7 of it (the oracle's, FP64 against extended): the tangent product only
+TANGENT_CASES = CASES + [
+    ("shear-quad-p5-hllc-br2-dense", lambda: _dense(P.ns_shear(n=3, order=5, flux=L.FLUX_HLLC, perturb=True))),
 ]
 
 
+def _sheared(n, order, visc):
+    """The shear layer on n x n parallelograms, opposite sides linked."""
+    _, prob, _ = P.ns_shear(n=n, order=order, flux=L.FLUX_HLLC, visc=visc, perturb=True)
+    n1 = n + 1
+    jj, ii = np.meshgrid(np.arange(n1), np.arange(n1), indexing="ij")
+    node = jj * n1 + ii
+    xy = np.stack([ii / n + 0.3 * jj / n, jj / n], -1).reshape(-1, 2)
+    quads = np.stack([node[:-1, :-1], node[:-1, 1:], node[1:, 1:], node[1:, :-1]], -1).reshape(-1, 4)
+    links = [list(zip(node[:, n].tolist(), node[:, 0].tolist())), list(zip(node[n].tolist(), node[0].tolist()))]
+    mesh = L.Mesh.from_arrays(L.ELEM_QUADRANGLE, order, xy, quads, periodic=links)
+    assert mesh.Fb == 0
+    return mesh, prob, P.shear_layer_primitive(mesh.field("quad_coord").reshape(mesh.E, mesh.nq, 2), 0.1, True)
+
+
 def _dense(case):
-    """The same case on the dense matrix-core kernels (hexahedra default to the sum-factorised
-    stage kernels and their adjoint)."""
+    """The same case on the dense matrix-core kernels (hexahedra and quadrangles default to the
+    sum-factorised stage kernels and their adjoint)."""
     mesh, prob, prim = case
     prob.kernels = L.KERNELS_DENSE
     return mesh, prob, prim
@@ -77,7 +107,7 @@ def test_residual_vjp_dot_product(name, make):
     assert abs(adj - fd_cpu) <= 1e-7 * abs(adj), (adj, fd_cpu)
 
 
-@pytest.mark.parametrize("name,make", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("name,make", TANGENT_CASES, ids=[c[0] for c in TANGENT_CASES])
 def test_residual_vjp_tangent_dot_product(name, make):
     """<J v, w> with J v from the oracle's tangent-linear build (forward-mode numbers through the
     oracle's passes, no difference quotient) equals <v, J^T w> from the GPU adjoint kernels to

@@ -209,3 +209,56 @@ def test_sum_factorised_and_dense_hexahedron_kernels_agree(order, visc):
     x.step(dt, 3)
     u1 = s_dn.get_state()
     fp64_parity(s_sf.get_state(), u1, x.get_state(), u1, mesh.dim)
+
+
+def _large(element, order, n):
+    if element == L.ELEM_TRIANGLE:
+        return L.Mesh.split(order, (n, n), (0.0, 0.0), (1.0, 1.0), 1.0, 7)
+    if element == L.ELEM_TETRAHEDRON:
+        return P.tet_box(n=n, order=order)
+    return L.Mesh(element, order, (n, n), (0.0, 0.0), (1.0, 1.0))
+
+
+@pytest.mark.parametrize("kind", ["ns", "av"])
+@pytest.mark.parametrize("element,order,n,mixed", [(L.ELEM_QUADRANGLE, 3, 45, False), (L.ELEM_QUADRANGLE, 3, 46, False),
+                                                   (L.ELEM_QUADRANGLE, 4, 46, False), (L.ELEM_QUADRANGLE, 3, 46, True),
+                                                   (L.ELEM_QUADRANGLE, 3, 65, True), (L.ELEM_TRIANGLE, 1, 46, False),
+                                                   (L.ELEM_TRIANGLE, 2, 46, False), (L.ELEM_TETRAHEDRON, 1, 9, False)])
+def test_dense_kernels_around_the_grid_where_their_wavefronts_change(element, order, n, mixed, kind):
+    """Gradient and residual kernels on grids below and above 1024 workgroups (other tests' meshes are far
+    below): residual and 2 steps against the FP64 vector kernels, FP64 at the parity bar, mixed precision
+    in L2 at the bar of its own tests (1e-6)."""
+    print(f"dense element {element} P{order} n={n} mixed={mixed} {kind}", flush=True)
+    mesh = _large(element, order, n)
+    kw = dict(cp=3.5, cv=2.5, convective_flux=L.FLUX_HLLC)
+    if kind == "ns":
+        kw.update(equation=L.EQ_NS, viscous_flux=L.VISC_BR2, transport=L.TRANSPORT_CONSTANT, dynamic_viscosity=0.01)
+    else:
+        kw.update(equation=L.EQ_EULER, shock_capturing=L.SHOCK_ARTIFICIAL_VISCOSITY, empirical_tolerance=4.0)
+    prob = L.problem_desc(**kw)
+    x = mesh.field("quad_coord").reshape(mesh.E, mesh.nq, mesh.dim)
+    prim = np.zeros((mesh.E, mesh.nq, mesh.nv))
+    prim[..., 0] = 1.0 + 0.2 * np.sin(2 * np.pi * x[..., 0])
+    prim[..., 1], prim[..., 2] = 0.3, 0.1 * np.cos(2 * np.pi * x[..., 1])
+    prim[..., -1] = 1.0 + 0.1 * np.cos(2 * np.pi * x[..., 0])
+    v = L.Solver(P.with_kernels(prob, L.KERNELS_VECTOR), mesh)
+    v.set_initial_primitive(prim)
+    dense = P.with_kernels(prob, L.KERNELS_DENSE)
+    dense.precision = L.PREC_MIXED if mixed else L.PREC_FP64
+    s = L.Solver(dense, mesh)
+    u0 = v.get_state()
+    s.set_state(u0)
+    if not mixed:
+        assert P.parity_error(s.residual(), v.residual(), u0, mesh.dim) <= 1e-11
+    dt = v.compute_dt(0.1)
+    rs, _, ts = s.step(dt, 2)
+    rv, _, tv = v.step(dt, 2)
+    assert ts == tv == 2
+    a, b = s.get_state(), v.get_state()
+    if mixed:
+        assert np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(b)
+    else:
+        assert np.abs(rs - rv).max() <= 1e-10 * np.abs(rv).max()
+        assert P.parity_error(a, b, b, mesh.dim) <= TOL
+    s.close()
+    v.close()
