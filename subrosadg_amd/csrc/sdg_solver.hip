@@ -691,12 +691,16 @@ int sdg_create(const sdg_problem_desc* problem, const sdg_mesh* mesh_handle, sdg
   // P2-P4 (FP64 or mixed), else the FP64 vector kernels
   const bool tensor_av = ctx->av && tensor && tensor_size;
   const bool av_vector = ctx->av && problem->equation == SDG_EQ_COMPRESSIBLE_NS && !tensor_av;
-  // Tetrahedra P1, Navier-Stokes: a basis of 4 leaves most of a 16 x 16 tile empty, and on a small mesh
-  // the vector kernels' two launches a stage beat the matrix-core kernels' three (1296 elements: 79
-  // against 89 us a step; 2058 elements: 124 against 98)
-  const bool small_p1 = r.type == SDG_ELEM_TETRAHEDRON && r.order == 1 && mesh.elements <= 1536 &&
-                        problem->equation == SDG_EQ_COMPRESSIBLE_NS && problem->kernels == SDG_KERNELS_AUTO;
-  if (!selectLaunchers(r.type, r.order, force_vector || av_vector || small_p1, mixed, ctx->launch,
+  // Tetrahedra P1 with a gradient pass (Navier-Stokes, artificial viscosity): a basis of 4 leaves most of a
+  // 16 x 16 tile empty, and between the grids on which the matrix-core kernels are wide (kWideGrid) and
+  // meshes that fill the card the vector kernels' two launches a stage are ahead of their three. us a step,
+  // matrix-core and vector kernels, Navier-Stokes (artificial viscosity within the same lines): 57.4 and 61.5
+  // at 384 elements, 64.9 and 63.4 at 750, 75.1 and 71.5 at 1296, 85.7 and 111 at 2058. Euler alone, one
+  // launch a stage either way, is ahead on the matrix-core kernels at every size (32.5 and 32.9 at 48,
+  // 50.5 and 80.5 at 6000).
+  const bool mid_p1 = r.type == SDG_ELEM_TETRAHEDRON && r.order == 1 && mesh.elements > 512 && mesh.elements <= 1536 &&
+                      (problem->equation == SDG_EQ_COMPRESSIBLE_NS || ctx->av) && problem->kernels == SDG_KERNELS_AUTO;
+  if (!selectLaunchers(r.type, r.order, force_vector || av_vector || mid_p1, mixed, ctx->launch,
                        tensor && (!ctx->av || tensor_av))) {
     delete ctx;
     return fail(nullptr, SDG_E_UNSUPPORTED,

@@ -1,6 +1,6 @@
-"""GPU parity on curved (high-order geometry) meshes and on tetrahedra: the vector kernels with
-per-point Jacobians and per-element mass inverses (Geometry.cpp:44-100) against the oracle, which
-consumes the same per-point tables. Residual, lifted gradient (Navier-Stokes) and 5 SSP-RK3 steps at
+"""GPU parity on curved (high-order geometry) meshes -- the vector kernels with per-point Jacobians and
+per-element mass inverses (Geometry.cpp:44-100) against the oracle, which consumes the same per-point
+tables -- and on tetrahedra (matrix-core and vector kernels) and pyramids. Residual, lifted gradient (Navier-Stokes) and 5 SSP-RK3 steps at
 the FP64 bar."""
 import numpy as np
 import pytest
@@ -95,27 +95,56 @@ def test_tetrahedra_parity(order):
     _check(mesh, _euler())
 
 
-@pytest.mark.parametrize("order,visc", [(2, L.VISC_BR2), (3, L.VISC_BR1)])
-def test_tetrahedra_navier_stokes_with_boundaries(order, visc):
+@pytest.mark.parametrize("order,visc,kernels", [(2, L.VISC_BR2, L.KERNELS_AUTO), (3, L.VISC_BR1, L.KERNELS_AUTO),
+                                                (4, L.VISC_BR2, L.KERNELS_AUTO), (4, L.VISC_BR1, L.KERNELS_AUTO)]
+                         + [(1, v, k) for v in (L.VISC_BR1, L.VISC_BR2)
+                            for k in (L.KERNELS_AUTO, L.KERNELS_DENSE, L.KERNELS_VECTOR)])
+def test_tetrahedra_navier_stokes_with_boundaries(order, visc, kernels):
     """Jittered tetrahedra of a box with far-field sides, Navier-Stokes."""
-    print(f"tetrahedra P{order} ns visc {visc} bounded", flush=True)
+    print(f"tetrahedra P{order} ns visc {visc} kernels {kernels} bounded", flush=True)
     mesh = P.tet_box(n=2, order=order, periodic=False, jitter=0.2)
     bprim = np.tile(np.array([1.0, 0.3, 0.0, 0.0, 1.0]), (mesh.Fb, mesh.nfq, 1))
-    _check(mesh, _ns(visc), bprim)
+    _check(mesh, P.with_kernels(_ns(visc), kernels), bprim)
 
 
+@pytest.mark.parametrize("n", [5, 7])
+@pytest.mark.parametrize("kind", ["br1", "br2", "av"])
+def test_tetrahedra_p1_families_agree(kind, n):
+    """750 and 2058 elements P1, where the automatic choice is the vector and the matrix-core kernels (48,
+    in the tests above, the latter): 3 steps against each other (two evaluations of one scheme in FP64)."""
+    print(f"tetrahedra P1 n={n} {kind}", flush=True)
+    mesh = P.tet_box(n=n, order=1, periodic=False, jitter=0.2)
+    prob = _ns(L.VISC_BR1 if kind == "br1" else L.VISC_BR2)
+    if kind == "av":
+        prob = L.problem_desc(equation=L.EQ_EULER, convective_flux=L.FLUX_HLLC, cp=3.5, cv=2.5, empirical_tolerance=4.0,
+                              shock_capturing=L.SHOCK_ARTIFICIAL_VISCOSITY)
+    bprim = np.tile(np.array([1.0, 0.3, 0.0, 0.0, 1.0]), (mesh.Fb, mesh.nfq, 1))
+    out = []
+    for kernels in (L.KERNELS_AUTO, L.KERNELS_DENSE, L.KERNELS_VECTOR):
+        s = L.Solver(P.with_kernels(prob, kernels), mesh)
+        s.set_initial_primitive(_smooth(mesh, 3))
+        s.set_boundary_primitive(bprim)
+        r = s.residual()
+        s.step(s.compute_dt(0.05), 3)
+        out.append((r, s.get_state()))
+        s.close()
+    for r, u in out[:2]:
+        assert P.parity_error(r, out[2][0], out[2][1], 3) <= 1e-11
+        assert P.parity_error(u, out[2][1], out[2][1], 3) <= 1e-12
 
-def test_tetrahedra_artificial_viscosity_parity():
-    """Euler with artificial viscosity on jittered tetrahedra (P2): node viscosities and the residual."""
-    print("tetrahedra P2 artificial viscosity", flush=True)
-    mesh = P.tet_box(n=2, order=2, jitter=0.2)
+
+@pytest.mark.parametrize("order,kernels", [(1, L.KERNELS_AUTO), (1, L.KERNELS_DENSE), (2, L.KERNELS_AUTO), (3, L.KERNELS_AUTO)])
+def test_tetrahedra_artificial_viscosity_parity(order, kernels):
+    """Euler with artificial viscosity on jittered tetrahedra: node viscosities and the residual."""
+    print(f"tetrahedra P{order} artificial viscosity kernels {kernels}", flush=True)
+    mesh = P.tet_box(n=2, order=order, jitter=0.2)
     prob = L.problem_desc(equation=L.EQ_EULER, convective_flux=L.FLUX_HLLC, cp=3.5, cv=2.5,
                           shock_capturing=L.SHOCK_ARTIFICIAL_VISCOSITY, empirical_tolerance=4.0)
     xq = mesh.field("quad_coord").reshape(mesh.E, mesh.nq, 3)
     # a steep but smooth front: a jump inside a P2 tetrahedron projects to negative face densities
     rho = 0.75 + 0.25 * np.tanh((0.47 - xq[..., 0]) / 0.03)
     prim = np.stack([rho, 0 * rho, 0 * rho, 0 * rho, 0 * rho + 1.0], axis=-1)
-    s = L.Solver(prob, mesh)
+    s = L.Solver(P.with_kernels(prob, kernels), mesh)
     s.set_initial_primitive(prim)
     o, x = O.Oracle(prob, mesh), O.Oracle(prob, mesh, extended=True)
     for k in (o, x):
