@@ -20,9 +20,10 @@ BOX = ((L.BC_RIEMANN_FARFIELD,) * 2, (L.BC_ADIABATIC_SLIP_WALL,) * 2)
 INOUT = ((L.BC_VELOCITY_INFLOW, L.BC_PRESSURE_OUTFLOW), (L.BC_ADIABATIC_SLIP_WALL,) * 2)
 HEXBOX = ((L.BC_RIEMANN_FARFIELD,) * 2, (L.BC_ADIABATIC_SLIP_WALL,) * 2, None)
 
+# triangles P1: on 5^2 cells and more Sod's jump turns the oracle's own steps NaN
 CASES = [
     ("quad", 1, None, 8), ("quad", 2, None, 6), ("quad", 3, None, 6), ("quad", 4, None, 4), ("quad", 5, None, 4),
-    ("quad", 3, BOX, 6), ("quad", 2, INOUT, 6), ("tri", 2, None, 5), ("tri", 3, None, 4),
+    ("quad", 3, BOX, 6), ("quad", 2, INOUT, 6), ("tri", 1, None, 4), ("tri", 2, None, 5), ("tri", 3, None, 4), ("tri", 4, None, 4),
     ("hex", 2, None, 3), ("hex", 3, HEXBOX, 3),
 ]
 

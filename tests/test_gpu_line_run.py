@@ -79,3 +79,57 @@ def test_nan_stop():
     _, nb, tb = b.step(dt, 50)
     assert na == nb == 1 and ta == tb < 50
     assert a.step(dt, 0)[2] == 0
+
+
+def test_calls_of_several_launches():
+    """A launch takes at most 4096 steps: a longer call is bit-identical to the same steps in two calls of
+    other lengths (trace parity, step count and state cross from one launch to the next)."""
+    (a, _), (b, _) = _pair(1, 8, False, True), _pair(1, 8, False, True)
+    dt = a.compute_dt(0.1)
+    ra, na, ta = a.step(dt, 4099)
+    _, n1, t1 = b.step(dt, 2050)
+    rb, n2, t2 = b.step(dt, 2049)
+    assert (na, n1, n2) == (0, 0, 0) and (ta, t1, t2) == (4099, 2050, 2049)
+    assert np.array_equal(ra, rb)
+    assert np.array_equal(a.get_state(), b.get_state())
+    assert np.array_equal(a.residual(), b.residual())
+
+
+def test_nan_stop_in_the_first_of_two_launches():
+    """The launch behind the one that stopped leaves state and step count alone."""
+    a, b = _pair(3, 80, True, False)
+    dt = 200.0 * a.compute_dt(1.0)
+    ra, na, ta = a.step(dt, 4100)
+    rb, nb, tb = b.step(dt, 50)
+    assert na == nb == 1 and ta == tb < 50
+    assert np.isnan(ra).all() and np.isnan(rb).all()
+    ua = a.get_state()
+    assert np.isnan(ua).any()
+    c, _ = _pair(3, 80, True, False)
+    c.step(dt, ta)
+    assert np.array_equal(c.get_state(), ua, equal_nan=True)
+
+
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("right", [True, False])
+def test_nan_stop_of_an_infinite_boundary_flux(order, right):
+    """An infinite flux at one end point alone: the end point's basis values are 1 and exact zeros, so it
+    makes the residual's modes NaN, and both launch modes stop after the same step."""
+    ends = (L.BC_RIEMANN_FARFIELD, L.BC_VELOCITY_INFLOW)
+    mesh = L.Mesh(L.ELEM_LINE, order, (5,), (0.0,), (1.0,), boundary=(ends if right else ends[::-1],))
+    prob = L.problem_desc(cp=3.5, cv=2.5, equation=L.EQ_EULER, convective_flux=L.FLUX_HLLC)
+    prim = np.zeros((mesh.E, mesh.nq, 3))
+    prim[..., 0], prim[..., 1], prim[..., 2] = 1.0, 0.1, 1.0
+    b = np.zeros((mesh.Fb, mesh.nfq, 3))
+    b[..., 0], b[..., 1], b[..., 2] = 1.0, 0.1, 1.0
+    end = (P.boundary_points(mesh)[..., 0] > 0.5) == right
+    b[end] = [1e200, -1e200, 1.0]
+    out = []
+    for launch in (L.LAUNCH_GRAPH, L.LAUNCH_EAGER):
+        p = L.ProblemDesc.from_buffer_copy(prob)
+        p.launch = launch
+        s = L.Solver(p, mesh)
+        s.set_initial_primitive(prim)
+        s.set_boundary_primitive(b)
+        out.append(s.step(1e-3, 6)[1:])
+    assert out[0] == out[1] == (1, 1)

@@ -1,8 +1,7 @@
 """Boussinesq source term on the GPU (SourceTerm.cpp:29-58): residual and 5-step parity with the
-oracle on every kernel family that carries it -- vector kernels (Euler and Navier-Stokes, small
-bases), matrix-core kernels (Euler and Navier-Stokes quadrangles, dense hexahedra) and the
-sum-factorised hexahedron kernels (the source formed at their nodes) --, the mixed mode, and the
-refusal of the adjoint."""
+oracle on every kernel family that carries it -- vector kernels, dense matrix-core kernels (workgroups
+of one, two and four wavefronts, simplices) and the sum-factorised quadrangle and hexahedron kernels
+(the source formed at their nodes) --, the mixed mode, and the refusal of the adjoint."""
 import numpy as np
 import pytest
 
@@ -16,20 +15,39 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-12
 GRAD_TOL = 5e-11
 
-CASES = [("euler-quad-p2-valu", L.ELEM_QUADRANGLE, 2, L.EQ_EULER, False),
-         ("euler-quad-p3-mfma", L.ELEM_QUADRANGLE, 3, L.EQ_EULER, False),
-         ("ns-quad-p2-valu", L.ELEM_QUADRANGLE, 2, L.EQ_NS, False),
-         ("ns-quad-p3-mfma", L.ELEM_QUADRANGLE, 3, L.EQ_NS, False),
-         ("ns-hex-p2-sumfact", L.ELEM_HEXAHEDRON, 2, L.EQ_NS, False),
-         ("ns-hex-p3-sumfact", L.ELEM_HEXAHEDRON, 3, L.EQ_NS, False),
-         ("ns-hex-p3-dense", L.ELEM_HEXAHEDRON, 3, L.EQ_NS, True)]
+AUTO, DENSE, VECTOR = L.KERNELS_AUTO, L.KERNELS_DENSE, L.KERNELS_VECTOR
+CASES = [("euler-quad-p2-sumfact", L.ELEM_QUADRANGLE, 2, L.EQ_EULER, AUTO),
+         ("euler-quad-p3-sumfact", L.ELEM_QUADRANGLE, 3, L.EQ_EULER, AUTO),
+         ("ns-quad-p2-sumfact", L.ELEM_QUADRANGLE, 2, L.EQ_NS, AUTO),
+         ("ns-quad-p3-sumfact", L.ELEM_QUADRANGLE, 3, L.EQ_NS, AUTO),
+         ("euler-quad-p2-vector", L.ELEM_QUADRANGLE, 2, L.EQ_EULER, VECTOR),
+         ("ns-quad-p2-vector", L.ELEM_QUADRANGLE, 2, L.EQ_NS, VECTOR),
+         ("euler-quad-p3-dense", L.ELEM_QUADRANGLE, 3, L.EQ_EULER, DENSE),
+         ("ns-quad-p3-dense", L.ELEM_QUADRANGLE, 3, L.EQ_NS, DENSE),
+         ("ns-quad-p4-dense", L.ELEM_QUADRANGLE, 4, L.EQ_NS, DENSE),
+         ("euler-tri-p3-dense", L.ELEM_TRIANGLE, 3, L.EQ_EULER, AUTO),
+         ("ns-tri-p2-dense", L.ELEM_TRIANGLE, 2, L.EQ_NS, AUTO),
+         ("ns-tet-p2-dense", L.ELEM_TETRAHEDRON, 2, L.EQ_NS, AUTO),
+         ("ns-hex-p2-sumfact", L.ELEM_HEXAHEDRON, 2, L.EQ_NS, AUTO),
+         ("ns-hex-p3-sumfact", L.ELEM_HEXAHEDRON, 3, L.EQ_NS, AUTO),
+         ("ns-hex-p3-dense", L.ELEM_HEXAHEDRON, 3, L.EQ_NS, DENSE)]
 
 
-@pytest.mark.parametrize("name,element,order,eq,dense", CASES, ids=[c[0] for c in CASES])
-def test_source_residual_and_step_parity(name, element, order, eq, dense):
+def _case(element, order, eq):
+    if element == L.ELEM_TRIANGLE:
+        _, prob = _box(L.ELEM_QUADRANGLE, order, 2, eq, beta=0.7, tref=0.98)
+        return L.Mesh.split(order, (3, 3), (0.0, 0.0), (1.0, 1.0), 1.0, 7), prob
+    if element == L.ELEM_TETRAHEDRON:
+        _, prob = _box(L.ELEM_HEXAHEDRON, order, 2, eq, beta=0.7, tref=0.98)
+        return P.tet_box(n=2, order=order), prob
+    return _box(element, order, 3 if element == L.ELEM_HEXAHEDRON else 4, eq, beta=0.7, tref=0.98)
+
+
+@pytest.mark.parametrize("name,element,order,eq,kernels", CASES, ids=[c[0] for c in CASES])
+def test_source_residual_and_step_parity(name, element, order, eq, kernels):
     print(f"source parity {name}", flush=True)
-    mesh, prob = _box(element, order, 3 if element == L.ELEM_HEXAHEDRON else 4, eq, beta=0.7, tref=0.98)
-    s = L.Solver(P.with_kernels(prob, L.KERNELS_DENSE) if dense else prob, mesh)
+    mesh, prob = _case(element, order, eq)
+    s = L.Solver(P.with_kernels(prob, kernels), mesh)
     s.set_initial_primitive(_wavy_primitive(mesh))
     u0 = s.get_state()
     o = O.Oracle(prob, mesh)
