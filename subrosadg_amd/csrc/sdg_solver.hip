@@ -544,6 +544,31 @@ void toReference(const sdg_ctx* ctx, const std::vector<double>& dev, double* ref
       for (int v = 0; v < nv; v++) ref[(e * nb + b) * nv + v] = dev[(e * nv + v) * nb + b];
 }
 
+// states of up to this many doubles are converted on the host: the bare copy of 18 KB takes 11 us, one
+// behind a kernel 23; 295 KB (36864 doubles) take 36 and 35, 1.2 MB 158 and 89
+constexpr int64_t kHostLayout = 32768;
+
+// src (device layout) -> the caller's array (reference layout), through tmp, a device buffer of its size.
+// Larger states are transposed by the device and the copy lands in the caller's array: a host
+// transposition of the 84 MB of 32^3 P3 hexahedra through a copy of its own took 33 ms, half a 50-step run.
+int readReference(sdg_ctx* ctx, const double* src, double* tmp, double* out) {
+  const int64_t n = static_cast<int64_t>(ctx->E) * ctx->nv * ctx->nb;
+  const size_t bytes = static_cast<size_t>(n) * sizeof(double);
+  if (n <= kHostLayout) {
+    std::vector<double> dev(static_cast<size_t>(n));
+    HIP_TRY(ctx, hipMemcpyAsync(dev.data(), src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    toReference(ctx, dev, out);
+    return SDG_OK;
+  }
+  hipLaunchKernelGGL(deviceToReferenceKernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, ctx->stream, src,
+                     tmp, ctx->E, ctx->nv, ctx->nb);
+  HIP_TRY(ctx, hipGetLastError());
+  HIP_TRY(ctx, hipMemcpyAsync(out, tmp, bytes, hipMemcpyDeviceToHost, ctx->stream));
+  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  return SDG_OK;
+}
+
 // Mixed-precision reference state: the domain mean of the conserved variables (mean over elements
 // of the element means) and its pressure.
 void updateReference(sdg_ctx* ctx, const double* ref) {
@@ -1231,20 +1256,11 @@ int sdg_set_state(sdg_ctx* ctx, const double* coefficients) {
   return SDG_OK;
 }
 
-// The device transposes the state into the residual output buffer, which holds nothing between
-// calls, and the copy lands in the caller's array: a host transposition of the 84 MB of 32^3 P3
-// hexahedra through a copy of its own took 33 ms, half a 50-step run.
+// The state passes through the residual output buffer, which holds nothing between calls.
 int sdg_get_state(sdg_ctx* ctx, double* coefficients) {
   if (!ctx || !coefficients) return fail(ctx, SDG_E_INVALID, "sdg_get_state: null argument");
   if (!ctx->has_state) return fail(ctx, SDG_E_STATE, "sdg_get_state: no state set");
-  const int64_t n = static_cast<int64_t>(ctx->E) * ctx->nv * ctx->nb;
-  hipLaunchKernelGGL(deviceToReferenceKernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, ctx->stream,
-                     ctx->U, ctx->Rout, ctx->E, ctx->nv, ctx->nb);
-  HIP_TRY(ctx, hipGetLastError());
-  HIP_TRY(ctx, hipMemcpyAsync(coefficients, ctx->Rout, static_cast<size_t>(n) * sizeof(double), hipMemcpyDeviceToHost,
-                              ctx->stream));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return SDG_OK;
+  return readReference(ctx, ctx->U, ctx->Rout, coefficients);
 }
 
 int sdg_set_initial_primitive(sdg_ctx* ctx, const double* prim) {
@@ -1342,22 +1358,23 @@ int sdg_residual(sdg_ctx* ctx, double* residual) {
   enqueueArtificialViscosity(ctx);
   enqueueStage(ctx, -1, 0.0, 1, nullptr);
   HIP_TRY(ctx, hipGetLastError());
+  // (the stage state buffer holds nothing between calls either; with a host copy beside the caller's array a
+  // call of 2.6 MB took 0.3 or 1.05 ms by what earlier calls had left of the heap)
+  if (!ctx->mixed || ctx->launch.tensor) return readReference(ctx, ctx->Rout, ctx->Us, residual);
   std::vector<double> dev(static_cast<size_t>(ctx->E) * ctx->nv * ctx->nb);
   HIP_TRY(ctx, hipMemcpyAsync(dev.data(), ctx->Rout, dev.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   // the dense mixed-precision kernels form R_psi = L^-1 R; return R = L R_psi (the sum-factorised
   // kernels write R itself)
-  if (ctx->mixed && !ctx->launch.tensor) {
-    const int nb = ctx->nb;
-    std::vector<double> t(nb);
-    for (size_t o = 0; o < dev.size(); o += nb) {
-      for (int i = 0; i < nb; i++) {
-        double acc = 0.0;
-        for (int j = 0; j <= i; j++) acc += ctx->h_chol[static_cast<size_t>(i) * nb + j] * dev[o + j];
-        t[i] = acc;
-      }
-      std::copy(t.begin(), t.end(), dev.begin() + static_cast<std::ptrdiff_t>(o));
+  const int nb = ctx->nb;
+  std::vector<double> t(nb);
+  for (size_t o = 0; o < dev.size(); o += nb) {
+    for (int i = 0; i < nb; i++) {
+      double acc = 0.0;
+      for (int j = 0; j <= i; j++) acc += ctx->h_chol[static_cast<size_t>(i) * nb + j] * dev[o + j];
+      t[i] = acc;
     }
+    std::copy(t.begin(), t.end(), dev.begin() + static_cast<std::ptrdiff_t>(o));
   }
   toReference(ctx, dev, residual);
   return SDG_OK;

@@ -266,3 +266,18 @@ def test_work_items_of_one_and_two_tiles(n, tiles_per_item, flux):
     b.step([dt], 3)
     u = s.get_state()
     assert P.parity_error(b.get_state(0).reshape(u.shape), u, u, 2) <= 1e-12
+
+
+@pytest.mark.parametrize("sizes", [(4, 5), (4, 5, 18)])
+def test_reads_on_both_sides_of_the_host_conversion(sizes):
+    """Batches below and above 8192 state values, converted on the host and on the device: every problem's
+    state comes back as set, to the rounding of the orthonormal basis' change of coefficients and back."""
+    meshes = [L.Mesh.split(p, (n, n), (-5.0, -5.0), (5.0, 5.0), 0.5, n) for p, n in zip((1, 3, 4), sizes)]
+    b = L.Batch(_euler(), meshes)
+    rng = np.random.default_rng(5)
+    states = [rng.standard_normal(k) for k in b.sizes]
+    for i, u in enumerate(states):
+        b.set_state(i, u)
+    assert (sum(b.sizes) > 8192) == (len(sizes) == 3)
+    for i, u in enumerate(states):
+        assert np.abs(b.get_state(i) - u).max() <= 1e-13 * np.abs(u).max()

@@ -262,3 +262,18 @@ def test_dense_kernels_around_the_grid_where_their_wavefronts_change(element, or
         assert P.parity_error(a, b, b, mesh.dim) <= TOL
     s.close()
     v.close()
+
+
+@pytest.mark.parametrize("n", [22, 23])
+def test_reads_on_both_sides_of_the_host_conversion(n):
+    """30976 and 33856 state values: the first are converted on the host, the second on the device. The
+    state comes back as it was set, the residual as the vector kernels' (another kernel family's own read)."""
+    mesh, prob, prim = P.euler_vortex(n=n, order=3)
+    s, v = L.Solver(prob, mesh), L.Solver(P.with_kernels(prob, L.KERNELS_VECTOR), mesh)
+    s.set_initial_primitive(prim)
+    u = s.get_state() * (1.0 + 1e-3 * np.random.default_rng(3).standard_normal(s.state_shape()))
+    s.set_state(u)
+    v.set_state(u)
+    assert np.array_equal(s.get_state(), u)
+    assert P.parity_error(s.residual(), v.residual(), u, 2) <= 1e-11
+    assert np.array_equal(s.get_state(), u)
