@@ -56,8 +56,8 @@ PROFILED_TRAFFIC = {("nsGradTensor", "fp64", 32, 3): (120703.0 * 2.0 + 204800.0 
 # the batched stage on the 48-problem workload: one launch per element variant (triangle and quadrangle,
 # P1-P4), FETCH_SIZE (x2.0) + WRITE_SIZE (x1.0) KiB per launch, summed over the 8 variants of a stage
 # (profiles/batch48_uneven_tri_quad_euler_kernels.md)
-PROFILED_BATCH_TRAFFIC = {"fp64": (568801.4) * 1024,
-                          "mixed": (494566.9) * 1024}
+PROFILED_BATCH_TRAFFIC = {"fp64": (523182.8) * 1024,
+                          "mixed": (445617.5) * 1024}
 
 
 def log(msg):
@@ -145,12 +145,11 @@ def tensor_path(mesh) -> bool:
 
 def roofline(kms, mesh, mode, n, kernels="auto"):
     """Roofline entry of the dominant kernel. kms: HIP-event averages of the gradient, face-flux and
-    residual kernels (and the monitor) on the solver's stream. `achieved`: the algorithmic bytes
-    B_alg per element-stage times the elements one launch processes, over the launch's duration
-    (B_alg counts the whole stage's state traffic, so this is the rate the stage would need if the
-    kernel were all of it). Also reported: the flop side of the same count (F_alg, the dense
-    formulation) and of the flops the sum-factorised kernels execute, and the whole stage (the
-    three kernels) against B_alg."""
+    residual kernels (and the monitor) on the solver's stream. `achieved`: where the launch's own HBM
+    bytes are known from a profile (`traffic`), these over its duration; elsewhere the stage's
+    algorithmic bytes (B_alg per element-stage, the state's traffic) over the duration of the stage's
+    three kernels. Also reported: the flop side of the same count (F_alg, the dense formulation) and of
+    the flops the sum-factorised kernels execute, and the whole stage against B_alg."""
     mixed = mode == "mixed"
     f_alg, b_alg = algorithmic_counts(mesh, mixed=mixed)
     tensor = tensor_path(mesh) and kernels == "auto"
@@ -164,9 +163,11 @@ def roofline(kms, mesh, mode, n, kernels="auto"):
     name, ms = names[k], float(kms[k])
     stage_ms = float(sum(kms[:3]))
     peak_f = PEAK_FP32_TFLOPS if mixed else PEAK_FP64_TFLOPS
-    achieved = b_alg * mesh.E / (ms * 1e-3) / 1e9
+    traffic = PROFILED_TRAFFIC.get((name, mode, n, mesh.order))
+    achieved = traffic / (ms * 1e-3) / 1e9 if traffic else b_alg * mesh.E / (stage_ms * 1e-3) / 1e9
     out = {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": achieved / PEAK_HBM_GBS,
-           "traffic": PROFILED_TRAFFIC.get((name, mode, n, mesh.order)), "kernel": name, "kernel_ms": ms,
+           "achieved_bytes": "profiled, of the kernel" if traffic else "algorithmic, of the stage",
+           "traffic": traffic, "kernel": name, "kernel_ms": ms,
            "algorithmic_bytes_per_element_stage": b_alg, "kernel_ms_all": [float(x) for x in kms],
            "kernel_ms_names": names + ["monitor"], "stage_ms": stage_ms,
            "stage_hbm_frac": b_alg * mesh.E / (stage_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
