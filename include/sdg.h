@@ -95,9 +95,11 @@ enum sdg_boundary {
 /* Kernel family of a single-problem context. AUTO: sum-factorised kernels on hexahedra P2-P4
  * (Navier-Stokes) and quadrangles P1-P5 (FP64), dense matrix-core kernels on the other matrix-core
  * sizes (quadrangles P3-P5 in mixed precision, hexahedra P2-P4 Euler, triangles and tetrahedra in
- * FP64), vector kernels elsewhere. DENSE keeps the dense matrix-core kernels where a size has them;
- * VECTOR runs the vector kernels for every size (FP64 only). All evaluate the same
- * operator; the choice exists to compare them. */
+ * FP64), vector kernels elsewhere and on 513 to 1536 tetrahedra P1 with a gradient pass. DENSE keeps
+ * the dense matrix-core kernels where a size has them; VECTOR runs the vector kernels for every size
+ * (FP64 only). All evaluate the same operator; the choice exists to compare them. Mixed precision pays
+ * on hexahedra and in the batch; on quadrangles FP64 is the faster mode in most cases (256^2 P3 with
+ * artificial viscosity 0.30 ms a step, mixed 0.50). */
 enum sdg_kernels { SDG_KERNELS_AUTO = 0, SDG_KERNELS_DENSE = 1, SDG_KERNELS_VECTOR = 2 };
 /* GRAPH: each sdg_step call replays whole steps from captured hipGraphs; EAGER: every kernel is
  * launched on the stream as it comes (same kernels, same results; on 1-D Euler meshes of up to 512

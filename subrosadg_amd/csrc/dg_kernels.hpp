@@ -188,7 +188,10 @@ struct StageArgs {
   float* Fv32;
   double* mon;    // E x NV monitor partials (last stage)
   int* status;    // [0] NaN stop flag, [1] steps taken, [2] the monitor's block counter; nullptr: no check
-  double c0, c1, c2dt;  // U <- c1 U + c0 Un + c2dt R Minv (TimeIntegration.cpp:181-198)
+  // U <- c1 U + c0 Un + c2dt R Minv (TimeIntegration.cpp:181-198). c0 is never zero; the kernels test it
+  // before they load Un because the compiler otherwise moves that load (quadrangles P3 with artificial
+  // viscosity, 192^2: 168 -> 170 registers, a wavefront less on each SIMD, 199 -> 210 us a step)
+  double c0, c1, c2dt;
   int last_stage;
   int mode;  // 0: stage update, 1: residual only
   // recording (matrix-core stage kernels): the updated state is also written to pool slot
@@ -1124,7 +1127,8 @@ __device__ __forceinline__ void blockVariableSums(const double* x, int64_t n, do
   }
 }
 
-// blocks of the monitor kernel: four loads a lane, so that a block is one round trip to memory
+// blocks of the monitor kernel: up to kMonitorBlocks of them take four loads a lane, one round trip to
+// memory; larger meshes take more loads a lane (32^3 hexahedra: ten)
 inline int monitorBlocks(int E, int nv) {
   const int64_t n = (static_cast<int64_t>(E) * nv + 4 * kThreads - 1) / (4 * kThreads);
   return n < kMonitorBlocks ? static_cast<int>(n) : kMonitorBlocks;

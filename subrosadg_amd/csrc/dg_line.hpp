@@ -256,6 +256,9 @@ __global__ __launch_bounds__(kLineMaxElements) void lineRunKernel(Geo g, Phys ph
 #pragma unroll
           for (int b = 0; b < N; b++) R[v][b] += g.Vf[s * N + b] * h[v];
       }
+      // The monitor's NaN test on the modes: an infinite flux at an end point meets the exact zero of the
+      // other end's mode, one inside makes the two end modes of opposite infinities, so that their sum is
+      // NaN where a node's value is.
       if (st == a.stages - 1) {
         int bad = 0;
         for (int v = 0; v < NV; v++) {
